@@ -22,7 +22,7 @@ STATUS = {0: "SQ_OK", 1: "SQ_ERR_IO", 2: "SQ_ERR_FORMAT", 3: "SQ_ERR_RANGE", 4: 
           6: "SQ_ERR_ALLOC", 7: "SQ_ERR_BREAKDOWN", 8: "SQ_ERR_DEVICE", 9: "SQ_ERR_STATE"}
 
 # every symbol include/sq_amd.h declares
-EXPORTS = ["sq_last_error", "sq_default_options", "sq_create_from_deck", "sq_destroy", "sq_get_info", "sq_set_veff",
+EXPORTS = ["sq_last_error", "sq_default_options", "sq_create_from_deck", "sq_destroy", "sq_get_info", "sq_resident_planes", "sq_set_veff",
            "sq_run", "sq_get_nodes_and_weights", "sq_get_lanczos", "sq_nodes_and_weights", "sq_last_timing",
            "sq_apply_h", "sq_apply_nonlocal", "sq_tridiag_nodes_weights", "sq_tridiag_nodes_weights_noalloc", "sq_tune_select", "sq_density_fermi_energy", "sq_synchronize",
            "sq_get_image", "sq_default_scf_options", "sq_scf", "sq_get_cell_field", "sq_set_veff_cell", "sq_xc",
@@ -106,6 +106,7 @@ def lib():
     L.sq_create_from_deck.argtypes = [C.c_char_p, C.c_char_p, C.POINTER(Options), C.POINTER(vp)]
     L.sq_destroy.argtypes = [vp]
     L.sq_get_info.argtypes = [vp, C.POINTER(Info)]
+    L.sq_resident_planes.argtypes = [vp, ip]
     L.sq_set_veff.argtypes = [vp, dp, C.c_double]
     L.sq_run.argtypes = [vp, C.c_int, C.c_int, lg, lg]
     L.sq_get_nodes_and_weights.argtypes = [vp, dp, dp, dp, dp]
@@ -211,6 +212,12 @@ class Context:
         I = Info()
         _check(lib().sq_get_info(self._h, C.byref(I)))
         return I
+
+    def resident_planes(self):
+        """Planes of the vector that FP64 passes keep in LDS; 0: the resident kernel is not used."""
+        p = C.c_int()
+        _check(lib().sq_resident_planes(self._h, C.byref(p)))
+        return p.value
 
     @property
     def nqp(self):

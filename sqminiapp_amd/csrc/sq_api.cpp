@@ -16,6 +16,7 @@
 #include "../../include/sq_amd.h"
 #include "sq_kernels.h"
 #include "sq_projectors.h"
+#include "sq_resident.h"
 #include "sq_system.h"
 
 using namespace sqamd;
@@ -74,6 +75,13 @@ struct sq_ctx {
     int bat_B = 0;
     int *probe_ids = nullptr;     // the autotuner's node set (one-node kernel form)
     float *bas32 = nullptr;       // column basis table of the batched kernel's FP32 form
+    // resident kernel (sq_resident.hip): grid (0: not used), planes of v in LDS, dynamic
+    // LDS, images trimmed to the projectors' reach and their padded tables
+    int res_grid = 0, res_nl = 0, res_n = 0;
+    size_t res_lds = 0, lds_limit = 0;
+    float res_rt2 = 0.f;
+    ResImage *res_img = nullptr;
+    double *res_tab = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     // device tables
@@ -151,7 +159,8 @@ void free_ctx(sq_ctx *c)
     void *ptrs[] = {c->img_dimp, c->rad64, c->rad32, c->img_rad, c->img_cen, c->chi64, c->chi32, c->img_lo, c->img_dim, c->img_off, c->img_atom, c->img_type, c->gamma,
                     c->cov_off, c->cov_img, c->diag64, c->diag32, c->c64, c->c32, c->scratch, c->a, c->b,
                     c->lam, c->w, c->lmin, c->lmax, c->qlws, c->status, c->partial, c->partial2, c->out,
-                    c->queue, c->nsteps, c->batches, c->probe_ids, c->bas32};
+                    c->queue, c->nsteps, c->batches, c->probe_ids, c->bas32, c->res_img,
+                    c->res_tab};
     void *scf_ptrs[] = {c->scf.rho, c->scf.rho_out, c->scf.b, c->scf.phi, c->scf.eps, c->scf.vxc, c->scf.veff, c->scf.r,
                         c->scf.p, c->scf.Ap, c->scf.f, c->scf.x_prev, c->scf.f_prev, c->scf.dX, c->scf.dF, c->scf.g,
                         c->scf.s, c->scf.part, c->scf.ku, c->scf.ky};
@@ -328,6 +337,7 @@ int create_device(sq_ctx *c, int device)
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, device));
     c->n_cu = prop.multiProcessorCount;
+    c->lds_limit = prop.sharedMemPerBlock;
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     for (auto &e : c->ev) HIP_TRY(hipEventCreate(&e));
     // the static workspace of sq_tridiag_nodes_weights_noalloc on this device
@@ -689,6 +699,156 @@ static int ensure_batches(sq_ctx *c, int B, long begin, long count)
     return SQ_OK;
 }
 
+// Radius past which no projector's radial function U_l dV_l exceeds eps of its
+// largest value (the spline between two knots stays within the knots' values
+// and slopes; past the core radius it rings down geometrically).
+static double projector_reach(const System &S, double eps)
+{
+    double reach = 0.0;
+    for (int t = 0; t < S.ntype; t++) {
+        const Pseudopotential &P = S.psd[t];
+        for (int l = 0; l <= P.lmax; l++) {
+            if (l == P.lloc) continue;
+            const std::vector<double> &y = P.s_udv[l].y, &yd = P.s_udv[l].yd;
+            double top = 0.0;
+            for (int k = 0; k < P.size; k++) top = std::max(top, std::fabs(y[k]));
+            for (int k = P.size - 2; k >= 0; k--) {
+                const double h = P.r[k + 1] - P.r[k];
+                if (std::max(std::fabs(y[k]), std::fabs(y[k + 1])) + h * std::max(std::fabs(yd[k]), std::fabs(yd[k + 1])) >
+                    eps * top) {
+                    reach = std::max(reach, P.r[k + 1]);
+                    break;
+                }
+            }
+        }
+    }
+    return reach;
+}
+
+static ResParams make_resident_params(const sq_ctx *c, int mode, long begin, long count)
+{
+    const System &S = c->sys;
+    ResParams P;
+    memset(&P, 0, sizeof P);
+    for (int d = 0; d < 3; d++) {
+        P.nloc[d] = S.nloc[d];
+        P.hw[d] = S.hw[d];
+        P.box0[d] = S.box[d];
+        P.box_n[d] = S.box[3 + d];
+        P.ext0[d] = S.ext0[d];
+        P.extn[d] = S.extn[d];
+        P.hgrid[d] = S.h[d];
+        P.range[d] = S.range[d];
+        for (int l = 0; l < 7; l++) P.cw[d][l] = S.coeff[d][l];
+    }
+    P.center = (((S.nloc[2] - 1) / 2) * S.nloc[1] + (S.nloc[1] - 1) / 2) * S.nloc[0] + (S.nloc[0] - 1) / 2;
+    P.nqp = S.nqp;
+    P.mode = mode;
+    P.n_images = c->res_n;
+    P.nl = c->res_nl;
+    P.node_begin = begin;
+    P.node_count = count;
+    P.rt2 = c->res_rt2;
+    P.img = c->res_img;
+    P.tab = c->res_tab;
+    P.gamma_ch = c->gamma;
+    P.diag_ext = c->diag64;
+    P.scratch = c->scratch;
+    P.out_a = c->a;
+    P.out_b = c->b;
+    P.status = c->status;
+    P.nsteps = c->nsteps;
+    P.queue = c->queue;
+    if (c->exit_tol > 0) {
+        P.exit_tol = c->exit_tol;
+        P.exit_lf = c->exit_lf;
+        P.exit_beta = c->exit_beta > 0 ? c->exit_beta : S.beta;
+        P.exit_min = std::max(2, c->exit_min);
+        P.exit_every = std::max(1, c->exit_every);
+    }
+    return P;
+}
+
+// The resident kernel's tables and shape.  It takes the cubes the column-
+// marching kernels take when their projectors are s+d, no side exceeds its
+// plane limit, no cube meets more images than it holds, and SQ_NO_RESIDENT is
+// not set (SQ_ZMARCH_WG, SQ_BATCH and SQ_BATCH_TRIP choose among the column-
+// marching kernels, which run where this one does not).  Box points past the
+// projectors' reach are dropped: at 2^-53 of the projector's largest value
+// they lie below the rounding of the sums they would enter.
+static int setup_resident(sq_ctx *c)
+{
+    const System &S = c->sys;
+    if (getenv("SQ_NO_RESIDENT")) return SQ_OK;
+    const int wg = resident_workgroup(S.nloc);
+    if (!c->zmarch || !c->zbatch || wg == 0 || c->img_cap > kResMaxImages) return SQ_OK;
+    if (S.ext_points() >= (int64_t)1 << 31 || S.n_nodes() >= (int64_t)1 << 31) return SQ_OK;
+    const double reach = projector_reach(S, std::ldexp(1.0, -53));
+    std::vector<ResImage> v;
+    for (size_t g = 0; g < S.images.size(); g++) {
+        const Image &im = S.images[g];
+        const double X[3] = {im.X0, im.Y0, im.Z0};
+        ResImage r;
+        memset(&r, 0, sizeof r);
+        bool empty = false;
+        for (int d = 0; d < 3; d++) {
+            const int lo = std::max(im.lo[d], (int)std::ceil((X[d] + S.range[d] - reach) / S.h[d]));
+            const int hi = std::min(im.hi[d], (int)std::floor((X[d] + S.range[d] + reach) / S.h[d]));
+            r.lo[d] = lo;
+            r.dim[d] = hi - lo + 1;
+            r.cen[d] = X[d];
+            empty = empty || hi < lo;
+            if (hi - lo >= 96) return SQ_OK;   // box origins and sizes are packed in bytes
+        }
+        if (empty) continue;
+        r.atom = im.atom;
+        r.type = im.type;
+        r.id = (int)g;
+        v.push_back(r);
+    }
+    std::stable_sort(v.begin(), v.end(), [](const ResImage &a, const ResImage &b) { return a.cen[2] < b.cen[2]; });
+    int64_t pairs = 0;
+    for (ResImage &r : v) {
+        r.off = (int)pairs;
+        pairs += (int64_t)r.dim[0] * r.dim[1] * (r.dim[2] + 2 * kResPad);
+        if (pairs >= (int64_t)1 << 30) return SQ_OK;   // pairs are indexed by int
+    }
+    // as many planes of v in LDS as fit, in whole chunks of planes: half the LDS for the
+    // small workgroup, two of which share a CU
+    const size_t limit = wg == 512 ? c->lds_limit / 2 : c->lds_limit;
+    int nl = S.nloc[2];
+    size_t total = 0, dynamic = 0;
+    for (; nl > 0; nl--) {
+        resident_lds(S.nloc, nl, &total, &dynamic);
+        if (total <= limit && (nl == S.nloc[2] || nl % 4 == 0)) break;
+    }
+    if (nl < 1 || v.empty()) return SQ_OK;
+    int rc;
+    if ((rc = dev_upload(&c->res_img, v.data(), v.size()))) return rc;
+    HIP_TRY(hipMalloc((void **)&c->res_tab, 2 * pairs * sizeof(double)));
+    HIP_TRY(launch_resident_tables(c->res_img, (int)v.size(), c->img_rad, c->img_lo, c->img_dim, c->rad64, c->res_tab,
+                                   c->stream));
+    c->res_n = (int)v.size();
+    c->res_nl = nl;
+    c->res_lds = dynamic;
+    c->res_rt2 = (float)(reach * reach);
+    const int occ = resident_occupancy(make_resident_params(c, SQ_NL_KB, 0, 1), dynamic);
+    if (occ > 0) c->res_grid = std::max(8, (c->n_cu * occ) & ~7);
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return SQ_OK;
+}
+
+// The resident kernel over rank-box nodes [begin, begin + count).
+static int launch_resident_pass(sq_ctx *c, int mode, long begin, long count)
+{
+    const ResParams P = make_resident_params(c, mode, begin, count);
+    c->last_exit = P.exit_tol > 0;
+    const int grid = (int)std::min<long>(c->res_grid, std::max<long>(8, (count + 7) & ~7L));
+    HIP_TRY(launch_zero_int(c->queue, 8, c->stream));
+    HIP_TRY(launch_resident(P, grid, c->res_lds, c->stream));
+    return SQ_OK;
+}
+
 // One Lanczos launch of configuration (B, shape or trip) on the probe's node
 // set, timed by HIP events on the context's stream.
 static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long nprobe, float *ms)
@@ -792,6 +952,8 @@ int finish_device_setup(sq_ctx *c)
                     scratch = std::max(scratch, (size_t)g * 3 * (S.nloc[2] + B - 1) * ncol * B * el);
                 }
     }
+    if (int rc = setup_resident(c)) return rc;
+    scratch = std::max(scratch, (size_t)c->res_grid * (S.nloc[2] - c->res_nl) * S.nloc[0] * S.nloc[1] * sizeof(double));
     HIP_TRY(hipMalloc(&c->scratch, scratch));
     if (!c->zmarch) return SQ_OK;
     for (int prec = 0; prec < 2; prec++) {
@@ -989,6 +1151,13 @@ int sq_get_info(sq_ctx *c, sq_info *I)
     return SQ_OK;
 }
 
+int sq_resident_planes(sq_ctx *c, int *planes)
+{
+    if (!c || !planes) return set_err(SQ_ERR_ARG, "null argument");
+    *planes = c->res_grid ? c->res_nl : 0;
+    return SQ_OK;
+}
+
 int sq_set_veff(sq_ctx *c, const double *field, double veff_const)
 {
     if (!c) return set_err(SQ_ERR_ARG, "null context");
@@ -1009,7 +1178,9 @@ int sq_run(sq_ctx *c, int mode, int precision, long begin, long count)
     c->have_run = false;
     HIP_TRY(hipEventRecord(c->ev[0], c->stream));
     c->last_exit = false;
-    if (c->zmarch && c->cfg_B[precision] > 1) {
+    if (c->res_grid && precision == SQ_FP64) {
+        if (int rc = launch_resident_pass(c, mode, begin, count)) return rc;
+    } else if (c->zmarch && c->cfg_B[precision] > 1) {
         const int B = c->cfg_B[precision];
         int rc = ensure_batches(c, B, begin, count);
         if (rc) return rc;
@@ -1628,7 +1799,9 @@ static int enqueue_sq_pass(sq_ctx *c, int mode, int precision)
     const long count = S.n_nodes();
     hipStream_t st = c->stream;
     c->last_exit = false;
-    if (c->zmarch && c->cfg_B[precision] > 1) {
+    if (c->res_grid && precision == SQ_FP64) {
+        if (int rc = launch_resident_pass(c, mode, 0, count)) return rc;
+    } else if (c->zmarch && c->cfg_B[precision] > 1) {
         const int B = c->cfg_B[precision];
         KParams P = make_batch_params(c, mode, precision, B, c->batches, c->n_batches);
         int grid = c->zb_grid[precision][B];
@@ -2067,7 +2240,17 @@ int sq_forces(sq_ctx *c, double *forces, double *f_local, double *f_nonlocal, sq
             const long cn = std::min(chunk, nlist - b0);
             HIP_TRY(hipMemcpyAsync(dids, ids.data() + b0, cn * sizeof(int), hipMemcpyHostToDevice, c->stream));
             bool exit_used = false;
-            if (c->zmarch) {
+            if (c->res_grid && prec == SQ_FP64) {
+                ResParams P = make_resident_params(c, SQ_NL_KB, 0, cn);
+                P.node_list = dids;
+                P.rec = drec;
+                P.rec_img = drimg;
+                P.rec_slots = slots;
+                exit_used = P.exit_tol > 0;
+                const int grid = (int)std::min<long>(c->res_grid, std::max<long>(8, (cn + 7) & ~7L));
+                HIP_TRY(launch_zero_int(c->queue, 8, c->stream));
+                HIP_TRY(launch_resident(P, grid, c->res_lds, c->stream));
+            } else if (c->zmarch) {
                 KParams P = make_params(c, SQ_NL_KB, prec, 0, cn, true);
                 P.node_list = dids;
                 P.rec = drec;
