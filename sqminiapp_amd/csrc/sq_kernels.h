@@ -84,7 +84,7 @@ hipError_t launch_basis_tables(const double *rad, int n_images, const int4 *lo, 
 hipError_t launch_apply(const KParams &P, long id, const double *x, double *y, int nonlocal_only, size_t lds,
                         hipStream_t st);
 hipError_t launch_ql(const double *a, const double *b, int n, int stride, long count, double *lam, double *w,
-                     double *lmin, double *lmax, int *status, double *ws, hipStream_t st, const int *nsteps = nullptr);
+                     double *lmin, double *lmax, int *status, hipStream_t st, const int *nsteps = nullptr);
 // QL of host-supplied device tridiagonals with its workspace in the library's
 // static device array (no allocation): the array's per-device address
 // (noalloc_scratch_init, with the device current), the bytes a call needs, and

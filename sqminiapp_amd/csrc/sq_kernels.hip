@@ -216,90 +216,145 @@ __global__ void __launch_bounds__(kWG) apply_kernel(KParams P, long id, const T 
     }
 }
 
-// Implicit QL of one tridiagonal per thread (TridiagEigenVecSolve_NodesAndWeights,
+// Implicit QL, one tridiagonal a lane (TridiagEigenVecSolve_NodesAndWeights,
 // lsdft_tools.cc:912-1026).  Only row 0 of the eigenvector matrix is carried:
 // the reference's rotations update each row of z independently, so row 0 -- the
 // one the weights w_i = z[0][i]^2 use -- is the same number sequence.
-__global__ void ql_kernel(const double *a, const double *bsub, int nmax, int stride, long count, double *lam, double *w,
-                          double *lmin, double *lmax, int *status, double *ws, const int *nsteps)
+//
+// Bound by the chain of one rotation (a square root and a division, about 500
+// clocks) times the rotations of a tridiagonal (5000 at n = 80), so what counts
+// is that nothing else joins the chain: d, e and z lie in LDS as [i][lane], the
+// next rotation's entries are read ahead, and the test for a small
+// off-diagonal, which the reference repeats from l on after every sweep, is
+// made inside the sweep, where d and e become final.  Only `lanes` lanes of a
+// wavefront work, so that a batch spreads over all SIMDs and few tridiagonals
+// wait for each other's sweeps.  16384 x n = 80: 11.4 ms with the three rows in
+// device memory and a scan before each sweep.
+__global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, const double *__restrict__ bsub, int nmax,
+                                                int stride, long count, int lanes, double *__restrict__ lam,
+                                                double *__restrict__ w, double *__restrict__ lmin,
+                                                double *__restrict__ lmax, int *__restrict__ status,
+                                                const int *__restrict__ nsteps)
 {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
+    extern __shared__ double rows[];   // d, e, z: [3][nmax][lanes]
+    const long t0 = (long)blockIdx.x * lanes;
+    const int mine = (int)min((long)lanes, count - t0), lane = threadIdx.x;
+    for (int q = lane; q < mine * nmax; q += 64) {
+        const int k = q / nmax, i = q - k * nmax;
+        rows[i * lanes + k] = a[(t0 + k) * stride + i];
+        rows[(nmax + i) * lanes + k] = bsub[(t0 + k) * stride + i];
+        rows[(2 * nmax + i) * lanes + k] = i == 0 ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    const long t = t0 + lane;
     // a node that stopped early has a Gauss rule of nsteps[t] nodes; the rest of
     // its row is padded with weight zero at its largest node
-    const int n = nsteps ? max(1, min(nmax, nsteps[t])) : nmax;
-    // d, e and row 0 of z live in a workspace laid out [i][thread] so that the
-    // threads of a wavefront touch consecutive addresses.
-    double *d = ws + t, *e = ws + (long)nmax * count + t, *z = ws + 2L * nmax * count + t;
-#define D(i) d[(long)(i) * count]
-#define EE(i) e[(long)(i) * count]
-#define Z(i) z[(long)(i) * count]
-    for (int i = 0; i < n; i++) {
-        D(i) = a[t * stride + i];
-        EE(i) = bsub[t * stride + i];
-        Z(i) = (i == 0) ? 1.0 : 0.0;
-    }
-    EE(n - 1) = 0.0;
-    int m, l, iter, i;
-    double s, r, p, g, f, dd, c, b;
-    for (l = 0; l <= n - 1; l++) {
-        iter = 0;
-        do {
-            for (m = l; m <= n - 2; m++) {
-                dd = fabs(D(m)) + fabs(D(m + 1));
-                if ((double)(fabs(EE(m)) + dd) == dd) break;
-            }
-            if (m != l) {
-                if (iter++ == 50) { status[t] = 5; return; }
-                g = (D(l + 1) - D(l)) / (2.0 * EE(l));
-                r = sqrt(g * g + 1.0);
-                g = D(m) - D(l) + EE(l) / (g + (g >= 0.0 ? fabs(r) : -fabs(r)));
-                s = c = 1.0;
-                p = 0.0;
-                for (i = m - 1; i >= l; i--) {
-                    f = s * EE(i);
-                    b = c * EE(i);
-                    EE(i + 1) = (r = sqrt(g * g + f * f));
+    int n = nmax, bad = 0;
+    if (lane < mine) {
+        if (nsteps) n = max(1, min(nmax, nsteps[t]));
+        double *const d = rows + lane, *const e = rows + nmax * lanes + lane, *const z = rows + 2 * nmax * lanes + lane;
+#define D(i) d[(i) * lanes]
+#define EE(i) e[(i) * lanes]
+#define Z(i) z[(i) * lanes]
+        EE(n - 1) = 0.0;
+        auto small = [](double ei, double di, double dn) {
+            const double dd = fabs(di) + fabs(dn);
+            return (double)(fabs(ei) + dd) == dd;
+        };
+        int next = -1;   // the first small off-diagonal from l on, where the last sweep found it
+        for (int l = 0; l < n && !bad; l++) {
+            for (int iter = 0;;) {
+                int m = next;
+                if (m < l) {
+                    m = l;
+                    for (double dm = D(l); m <= n - 2; m++) {
+                        const double dn = D(m + 1);
+                        if (small(EE(m), dm, dn)) break;
+                        dm = dn;
+                    }
+                    next = m;
+                }
+                if (m == l) break;
+                if (iter++ == 50) { bad = 5; break; }
+                const double el = EE(l);
+                double g = (D(l + 1) - D(l)) / (2.0 * el);
+                double r = sqrt(g * g + 1.0);
+                double dnext = D(m);   // d(i + 1) before rotation i
+                g = dnext - D(l) + el / (g + (g >= 0.0 ? fabs(r) : -fabs(r)));
+                double s = 1.0, c = 1.0, p = 0.0, znext = Z(m), dfinal = 0.0;
+                double di = D(m - 1), ei = EE(m - 1), zi = Z(m - 1);
+                int i = m - 1, above = m;   // above: the first small off-diagonal past l so far
+                for (;;) {
+                    // entries of rotation i - 1 (row 0 again on the last one)
+                    const int k = max(i - 1, 0);
+                    const double dk = D(k), ek = EE(k), zk = Z(k);
+                    const double f = s * ei, b = c * ei;
+                    r = sqrt(g * g + f * f);
+                    EE(i + 1) = r;
                     if (r == 0.0) {
-                        D(i + 1) -= p;
+                        D(i + 1) = dnext - p;
+                        Z(i + 1) = znext;
                         EE(m) = 0.0;
                         break;
                     }
                     s = f / r;
                     c = g / r;
-                    g = D(i + 1) - p;
-                    r = (D(i) - g) * s + 2.0 * c * b;
-                    D(i + 1) = g + (p = s * r);
-                    g = c * r - b;
-                    f = Z(i + 1);
-                    Z(i + 1) = s * Z(i) + c * f;
-                    Z(i) = c * Z(i) - s * f;
+                    g = dnext - p;
+                    const double rr = (di - g) * s + 2.0 * c * b;
+                    p = s * rr;
+                    const double dn = g + p;   // d(i + 1), final
+                    D(i + 1) = dn;
+                    g = c * rr - b;
+                    Z(i + 1) = s * zi + c * znext;
+                    znext = c * zi - s * znext;
+                    if (i + 1 < m && small(r, dn, dfinal)) above = i + 1;
+                    dfinal = dn;
+                    dnext = di;
+                    if (i == l) break;
+                    i--;
+                    di = dk;
+                    ei = ek;
+                    zi = zk;
                 }
-                if (r == 0.0 && i >= l) continue;
-                D(l) -= p;
+                if (r == 0.0) { next = -1; continue; }
+                const double dl = dnext - p;
+                D(l) = dl;
+                Z(l) = znext;
                 EE(l) = g;
                 EE(m) = 0.0;
+                next = above;
+                if (small(g, dl, dfinal)) break;
             }
-        } while (m != l);
-    }
-    double emin = D(0), emax = D(0);
-    for (i = 0; i < n; i++) {
-        const double di = D(i), zi = Z(i);
-        lam[t * nmax + i] = di;
-        w[t * nmax + i] = zi * zi;
-        if (di > emax) emax = di;
-        else if (di < emin) emin = di;
-    }
-    for (i = n; i < nmax; i++) {
-        lam[t * nmax + i] = emax;
-        w[t * nmax + i] = 0.0;
-    }
+        }
+        double emin = D(0), emax = D(0);
+        for (int i = 1; i < n; i++) {
+            const double di = D(i);
+            if (di > emax) emax = di;
+            else if (di < emin) emin = di;
+        }
+        status[t] = bad;
+        if (!bad) {
+            lmin[t] = emin;
+            lmax[t] = emax;
+            for (int i = n; i < nmax; i++) {
+                D(i) = emax;
+                Z(i) = 0.0;
+            }
+        }
 #undef D
 #undef EE
 #undef Z
-    lmin[t] = emin;
-    lmax[t] = emax;
-    status[t] = 0;
+    }
+    // a tridiagonal that did not converge leaves its outputs untouched
+    const unsigned long long failed = __ballot(bad != 0);
+    __syncthreads();
+    for (int q = lane; q < mine * nmax; q += 64) {
+        const int k = q / nmax, i = q - k * nmax;
+        if (failed >> k & 1) continue;
+        const double zi = rows[(2 * nmax + i) * lanes + k];
+        lam[(t0 + k) * nmax + i] = rows[i * lanes + k];
+        w[(t0 + k) * nmax + i] = zi * zi;
+    }
 }
 
 // ------------------------------------------------ density / Fermi / energy
@@ -431,14 +486,25 @@ hipError_t launch_apply(const KParams &P, long id, const double *x, double *y, i
     return hipGetLastError();
 }
 
+// Tridiagonals a wavefront of ql_kernel takes: as many as leave room for four
+// workgroups a CU, one a SIMD, and fewer where the batch is too small to give
+// every SIMD a wavefront otherwise.
+static int ql_lanes(int n, long count)
+{
+    int lanes = 16;
+    while (lanes > 1 && (size_t)lanes * 3 * n * sizeof(double) > 40960) lanes >>= 1;
+    while (lanes > 1 && count <= 512L * lanes) lanes >>= 1;
+    return lanes;
+}
+
 hipError_t launch_ql(const double *a, const double *b, int n, int stride, long count, double *lam, double *w,
-                     double *lmin, double *lmax, int *status, double *ws, hipStream_t st, const int *nsteps)
+                     double *lmin, double *lmax, int *status, hipStream_t st, const int *nsteps)
 {
     if (n < 1 || n > kMaxNqp || count <= 0) return hipErrorInvalidValue;
-    const int threads = 64;
-    const long blocks = (count + threads - 1) / threads;
-    hipLaunchKernelGGL(ql_kernel, dim3((unsigned)blocks), dim3(threads), 0, st, a, b, n, stride, count, lam, w, lmin,
-                       lmax, status, ws, nsteps);
+    const int lanes = ql_lanes(n, count);
+    const long blocks = (count + lanes - 1) / lanes;
+    hipLaunchKernelGGL(ql_kernel, dim3((unsigned)blocks), dim3(64), (size_t)lanes * 3 * n * sizeof(double), st, a, b, n,
+                       stride, count, lanes, lam, w, lmin, lmax, status, nsteps);
     return hipGetLastError();
 }
 
@@ -523,8 +589,9 @@ void *noalloc_scratch(int device)
     return g_scratch_dev[device];
 }
 
-// workspace layout: QL d, e and z row 0 [3][n][count] doubles | status[count] |
-// the index of the first failed tridiagonal (long long)
+// workspace layout: [3][n][count] doubles, the room of QL's three rows in device
+// memory (it keeps them in LDS now; the limit on a batch is the interface's) |
+// status[count] | the index of the first failed tridiagonal (long long)
 size_t noalloc_ql_bytes(int n, long count)
 {
     return align256((size_t)3 * n * count * sizeof(double)) + align256((size_t)count * sizeof(int)) + 256;
@@ -553,11 +620,10 @@ hipError_t launch_ql_noalloc(void *ws, const double *a, const double *b, int n, 
     if (!ws || n < 1 || n > kMaxNqp || count <= 0 || noalloc_ql_bytes(n, count) > kNoAllocScratchBytes)
         return hipErrorInvalidValue;
     unsigned char *base = static_cast<unsigned char *>(ws);
-    double *d = reinterpret_cast<double *>(base);
     int *status = reinterpret_cast<int *>(base + align256((size_t)3 * n * count * sizeof(double)));
     long long *bad = reinterpret_cast<long long *>(reinterpret_cast<unsigned char *>(status) +
                                                    align256((size_t)count * sizeof(int)));
-    hipError_t e = launch_ql(a, b, n, n, count, lam, w, lmin, lmax, status, d, st);
+    hipError_t e = launch_ql(a, b, n, n, count, lam, w, lmin, lmax, status, st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(first_failure, dim3(1), dim3(256), 0, st, status, count, bad);
     *first_bad = bad;
