@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <climits>
 #include <mutex>
 
@@ -216,20 +217,53 @@ __global__ void __launch_bounds__(kWG) apply_kernel(KParams P, long id, const T 
     }
 }
 
+// r = sqrt(g g + f f), s = f / r, c = g / r, each correctly rounded as the
+// operators round them.  One approximate 1/sqrt serves all three: coupled
+// Newton steps (Goldschmidt) give sqrt(x) and 1/(2 sqrt(x)), two residual
+// corrections round the root, one more Newton step rounds 1/r, and the residual
+// of each quotient rounds it (Markstein, IBM J. Res. Dev. 34, 1990).  That needs
+// operands away from the ends of the exponent range; others (zeros among them)
+// take the operators, whose range scaling costs a third of the chain.
+__device__ __forceinline__ void rotation(double f, double g, double &r, double &s, double &c)
+{
+    const double x = g * g + f * f;
+    const double af = fabs(f), ag = fabs(g);
+    if (fmin(af, ag) > 0x1p-300 && fmax(af, ag) < 0x1p300) {
+        const double y = __builtin_amdgcn_rsq(x);
+        double q = x * y, h = 0.5 * y;
+        const double t = fma(-h, q, 0.5);
+        q = fma(q, t, q);
+        h = fma(h, t, h);
+        q = fma(fma(-q, q, x), h, q);
+        r = fma(fma(-q, q, x), h, q);
+        h = h + h;
+        h = fma(fma(-r, h, 1.0), h, h);
+        h = fma(fma(-r, h, 1.0), h, h);
+        const double qf = f * h, qg = g * h;
+        s = fma(fma(-r, qf, f), h, qf);
+        c = fma(fma(-r, qg, g), h, qg);
+    } else {
+        r = sqrt(x);
+        s = f / r;
+        c = g / r;
+    }
+}
+
 // Implicit QL, one tridiagonal a lane (TridiagEigenVecSolve_NodesAndWeights,
 // lsdft_tools.cc:912-1026).  Only row 0 of the eigenvector matrix is carried:
 // the reference's rotations update each row of z independently, so row 0 -- the
 // one the weights w_i = z[0][i]^2 use -- is the same number sequence.
 //
-// Bound by the chain of one rotation (a square root and a division, about 500
+// Bound by the chain of one rotation (rotation(), about 400
 // clocks) times the rotations of a tridiagonal (5000 at n = 80), so what counts
 // is that nothing else joins the chain: d, e and z lie in LDS as [i][lane], the
 // next rotation's entries are read ahead, and the test for a small
 // off-diagonal, which the reference repeats from l on after every sweep, is
 // made inside the sweep, where d and e become final.  Only `lanes` lanes of a
 // wavefront work, so that a batch spreads over all SIMDs and few tridiagonals
-// wait for each other's sweeps.  16384 x n = 80: 11.4 ms with the three rows in
-// device memory and a scan before each sweep.
+// wait for each other's sweeps.  16384 x n = 80: 3.1 ms; 11.4 with the three rows
+// in device memory and a scan before each sweep, 3.3 with the operators in place
+// of rotation().
 __global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, const double *__restrict__ bsub, int nmax,
                                                 int stride, long count, int lanes, double *__restrict__ lam,
                                                 double *__restrict__ w, double *__restrict__ lmin,
@@ -289,7 +323,7 @@ __global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, co
                     const int k = max(i - 1, 0);
                     const double dk = D(k), ek = EE(k), zk = Z(k);
                     const double f = s * ei, b = c * ei;
-                    r = sqrt(g * g + f * f);
+                    rotation(f, g, r, s, c);
                     EE(i + 1) = r;
                     if (r == 0.0) {
                         D(i + 1) = dnext - p;
@@ -297,8 +331,6 @@ __global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, co
                         EE(m) = 0.0;
                         break;
                     }
-                    s = f / r;
-                    c = g / r;
                     g = dnext - p;
                     const double rr = (di - g) * s + 2.0 * c * b;
                     p = s * rr;
@@ -486,14 +518,18 @@ hipError_t launch_apply(const KParams &P, long id, const double *x, double *y, i
     return hipGetLastError();
 }
 
-// Tridiagonals a wavefront of ql_kernel takes: as many as leave room for four
-// workgroups a CU, one a SIMD, and fewer where the batch is too small to give
-// every SIMD a wavefront otherwise.
+// Tridiagonals a wavefront of ql_kernel takes: the fewest with which every
+// wavefront has a CU to itself (n = 80: 33 take 2.6 ms one a wavefront and 2.9
+// sixteen a wavefront; 3840 take 3.65 sixteen a wavefront and 4.4 eight; 7872
+// take 3.9 and 4.7 with 32 and 16), else 16 on four wavefronts a CU (16384:
+// 3.1, against 3.6 with 32), as far as their rows fit LDS.
 static int ql_lanes(int n, long count)
 {
-    int lanes = 16;
-    while (lanes > 1 && (size_t)lanes * 3 * n * sizeof(double) > 40960) lanes >>= 1;
-    while (lanes > 1 && count <= 512L * lanes) lanes >>= 1;
+    const size_t row = (size_t)3 * n * sizeof(double);
+    int lanes = 1;
+    while (lanes < 32 && (count + lanes - 1) / lanes > 256) lanes <<= 1;
+    if ((count + lanes - 1) / lanes > 256) lanes = 16;
+    while (lanes > 1 && lanes * row > (lanes > 16 ? 65536 : 40960)) lanes >>= 1;
     return lanes;
 }
 
@@ -503,8 +539,11 @@ hipError_t launch_ql(const double *a, const double *b, int n, int stride, long c
     if (n < 1 || n > kMaxNqp || count <= 0) return hipErrorInvalidValue;
     const int lanes = ql_lanes(n, count);
     const long blocks = (count + lanes - 1) / lanes;
-    hipLaunchKernelGGL(ql_kernel, dim3((unsigned)blocks), dim3(64), (size_t)lanes * 3 * n * sizeof(double), st, a, b, n,
-                       stride, count, lanes, lam, w, lmin, lmax, status, nsteps);
+    // LDS for the rows, and no less than keeps a CU from taking more workgroups than its share
+    const size_t rows = (size_t)lanes * 3 * n * sizeof(double);
+    const size_t share = blocks > 512 ? 40960 : 65536;
+    hipLaunchKernelGGL(ql_kernel, dim3((unsigned)blocks), dim3(64), std::max(rows, share), st, a, b, n, stride, count,
+                       lanes, lam, w, lmin, lmax, status, nsteps);
     return hipGetLastError();
 }
 
