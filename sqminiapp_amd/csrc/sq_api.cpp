@@ -37,7 +37,7 @@ int set_err(int code, const std::string &msg)
             return set_err(SQ_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_));             \
     } while (0)
 
-constexpr int kRedBlocks = 512;
+constexpr int kRedBlocks = kRedBlocksDev;
 }  // namespace
 
 namespace sqamd {
@@ -104,7 +104,8 @@ struct sq_ctx {
     double *a = nullptr, *b = nullptr, *lam = nullptr, *w = nullptr, *lmin = nullptr, *lmax = nullptr;
     int *status = nullptr;
     int *queue = nullptr, *nsteps = nullptr;   // z-march work queue (8 counters); Gauss nodes per node
-    double *partial = nullptr, *partial2 = nullptr, *out = nullptr;
+    double *partial = nullptr, *out = nullptr;
+    BisState *bis = nullptr;      // Fermi bisection
     // per-node early exit of the z-march kernel (exit_tol <= 0: off)
     double exit_tol = 0, exit_lf = 0, exit_beta = 0;
     int exit_min = 30, exit_every = 5;
@@ -158,7 +159,7 @@ void free_ctx(sq_ctx *c)
     if (!c) return;
     void *ptrs[] = {c->img_dimp, c->rad64, c->rad32, c->img_rad, c->img_cen, c->chi64, c->chi32, c->img_lo, c->img_dim, c->img_off, c->img_atom, c->img_type, c->gamma,
                     c->cov_off, c->cov_img, c->diag64, c->diag32, c->c64, c->c32, c->scratch, c->a, c->b,
-                    c->lam, c->w, c->lmin, c->lmax, c->status, c->partial, c->partial2, c->out,
+                    c->lam, c->w, c->lmin, c->lmax, c->status, c->partial, c->bis, c->out,
                     c->queue, c->nsteps, c->batches, c->probe_ids, c->bas32, c->res_img,
                     c->res_tab};
     void *scf_ptrs[] = {c->scf.rho, c->scf.rho_out, c->scf.b, c->scf.phi, c->scf.eps, c->scf.vxc, c->scf.veff, c->scf.r,
@@ -422,8 +423,8 @@ int create_device(sq_ctx *c, int device)
     HIP_TRY(hipMalloc((void **)&c->lmin, nn * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->lmax, nn * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->status, std::max<int64_t>(nn, 1) * sizeof(int)));
-    HIP_TRY(hipMalloc((void **)&c->partial, kRedBlocks * sizeof(double)));
-    HIP_TRY(hipMalloc((void **)&c->partial2, kRedBlocks * sizeof(double)));
+    HIP_TRY(hipMalloc((void **)&c->partial, 3 * kRedBlocks * sizeof(double)));
+    HIP_TRY(hipMalloc((void **)&c->bis, 2 * sizeof(BisState)));
     HIP_TRY(hipMalloc((void **)&c->out, 4 * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->queue, 8 * sizeof(int)));
     HIP_TRY(hipMalloc((void **)&c->nsteps, std::max<int64_t>(1, nn) * sizeof(int)));
@@ -1420,37 +1421,26 @@ static int density_device(sq_ctx *c, double nelec, double beta, double *lambda_f
     if (beta <= 0) beta = S.beta;
     HIP_TRY(hipSetDevice(c->device));
     const long nq = nn * S.nqp;
-    double range[2];
+    // bisection on the device (fermi_count): the counts that usually suffice at once, more
+    // only if it has not stopped
     HIP_TRY(launch_lam_range(c->lmin, c->lmax, nn, c->out, c->stream));
-    HIP_TRY(hipMemcpyAsync(range, c->out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    double lo = range[0] - 1.0, hi = range[1] + 1.0;
-    auto count_at = [&](double lf, double *res) -> int {
-        HIP_TRY(launch_occupation(c->lam, c->w, nq, beta, lf, c->partial, kRedBlocks, c->out, c->stream));
-        HIP_TRY(hipMemcpyAsync(res, c->out, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    BisState b;
+    memset(&b, 0, sizeof b);
+    for (int k = -2, upto = 60; !b.done; upto += 48) {
+        for (; k <= upto; k++)
+            HIP_TRY(launch_fermi_count(c->lam, c->w, nq, beta, nelec, c->out, k, c->bis, c->partial, c->stream));
+        HIP_TRY(hipMemcpyAsync(&b, c->bis + ((k - 1) & 1), sizeof b, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
-        return SQ_OK;
-    };
-    double glo, ghi;
-    int rc;
-    if ((rc = count_at(lo, &glo)) || (rc = count_at(hi, &ghi))) return rc;
-    if (glo - nelec > 0 || ghi - nelec < 0) return set_err(SQ_ERR_RANGE, "Fermi level not bracketed by the spectrum");
-    // bisection on [lambda_min - 1, lambda_max + 1] to 1e-14 (relative), at most 200 halvings
-    for (int it = 0; it < 200; it++) {
-        double mid = 0.5 * (lo + hi);
-        if (hi - lo <= 1e-14 * (std::fabs(mid) > 1.0 ? std::fabs(mid) : 1.0)) break;
-        double g;
-        if ((rc = count_at(mid, &g))) return rc;
-        if (g - nelec > 0) hi = mid;
-        else lo = mid;
+        if (b.done) {
+            if (b.bad) return set_err(SQ_ERR_RANGE, "Fermi level not bracketed by the spectrum");
+            HIP_TRY(launch_density_energy(c->lam, c->w, nn, S.nqp, beta, &c->bis[(k - 1) & 1].lf, 2.0 / S.dV, drho, c->partial,
+                                          c->out, c->stream));
+        }
     }
-    const double lf = 0.5 * (lo + hi);
     double res[2];
-    HIP_TRY(launch_density_energy(c->lam, c->w, nn, S.nqp, beta, lf, 2.0 / S.dV, drho, c->partial, c->partial2,
-                                  kRedBlocks, c->out, c->stream));
     HIP_TRY(hipMemcpyAsync(res, c->out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    *lambda_f = lf;
+    *lambda_f = b.lf;
     *e_band = res[0];
     *minus_ts = res[1];
     return SQ_OK;
@@ -1539,7 +1529,7 @@ static int scf_alloc(sq_ctx *c, int hist)
         if (!e) HIP_TRY(hipEventCreate(&e));
     HIP_TRY(hipMalloc((void **)&F.g, std::max(1, hist) * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&F.s, 16 * sizeof(double)));
-    HIP_TRY(hipMalloc((void **)&F.part, kRedBlocks * sizeof(double)));
+    HIP_TRY(hipMalloc((void **)&F.part, 2 * kRedBlocks * sizeof(double)));
     F.ng = ng;
     F.hist = hist;
     if (F.have_b) HIP_TRY(hipMemcpy(F.b, F.host_b.data(), ng * sizeof(double), hipMemcpyHostToDevice));
@@ -1600,26 +1590,23 @@ static int scf_poisson(sq_ctx *c, const double *f, double tol, int max_it, int *
     double rr = 0.0;
     HIP_TRY(hipMemcpyAsync(&rr, F.s, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    // One CG step is seven launches (stencil, two two-stage dots, two updates),
-    // all on fixed buffers with their scalars on the device: four steps are
-    // captured once as a graph and replayed between the host's convergence
-    // checks (SQ_NO_GRAPHS set: launched one by one, the same kernels in the
-    // same order).
-    auto cg_step = [&]() -> int {
-        HIP_TRY(launch_lap_periodic(F.p, F.Ap, G, S.order, sc, c->stream));
-        if (int r2 = scf_dot(c, F.p, F.Ap, 1, nullptr)) return r2;
-        HIP_TRY(launch_cg_xr(F.phi, F.r, F.p, F.Ap, F.s, n, c->stream));
-        if (int r2 = scf_dot(c, F.r, F.r, 2, nullptr)) return r2;
-        HIP_TRY(launch_cg_p(F.p, F.r, F.s, n, c->stream));
+    // One CG step is three launches on fixed buffers with their scalars on the
+    // device: four steps are captured once as a graph and replayed between the
+    // host's convergence checks (SQ_NO_GRAPHS set: launched one by one, the same
+    // kernels in the same order).  <r,r> alternates between slots 0 and 2.
+    auto cg_step = [&](int k) -> int {
+        HIP_TRY(launch_cg_step(F.phi, F.r, F.p, F.Ap, F.s + 2 * (k & 1), F.s + 2 - 2 * (k & 1), 0.0, G, S.order, sc, F.part,
+                               kRedBlocks, c->stream));
         return SQ_OK;
     };
     const bool graphs = getenv("SQ_NO_GRAPHS") == nullptr;
     while (rr > stop && it < max_it) {
+        const double *at = F.s;   // <r,r> after the steps
         if (graphs && it + 4 <= max_it) {
             if (!F.cg_exec) {
                 HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
                 int rc2 = SQ_OK;
-                for (int k = 0; k < 4 && !rc2; k++) rc2 = cg_step();
+                for (int k = 0; k < 4 && !rc2; k++) rc2 = cg_step(k);
                 hipGraph_t g = nullptr;
                 const hipError_t e = hipStreamEndCapture(c->stream, &g);
                 if (rc2) { if (g) (void)hipGraphDestroy(g); return rc2; }
@@ -1630,10 +1617,12 @@ static int scf_poisson(sq_ctx *c, const double *f, double tol, int max_it, int *
             HIP_TRY(hipGraphLaunch(F.cg_exec, c->stream));
             it += 4;
         } else {
-            for (int k = 0; k < 4 && it < max_it; k++, it++)
-                if ((rc = cg_step())) return rc;
+            int k = 0;
+            for (; k < 4 && it < max_it; k++, it++)
+                if ((rc = cg_step(k))) return rc;
+            at = F.s + 2 * (k & 1);
         }
-        HIP_TRY(hipMemcpyAsync(&rr, F.s, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipMemcpyAsync(&rr, at, sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
     }
     if (!(rr <= stop)) return set_err(SQ_ERR_RANGE, "Poisson: conjugate gradients did not reach TOL_POISSON");
@@ -1669,12 +1658,8 @@ static int scf_kerker(sq_ctx *c, const double *u, double *y, double k0, int *ite
     int it = 0;
     while (rr > stop && it < 2000) {
         for (int k = 0; k < 4; k++, it++) {
-            HIP_TRY(launch_lap_periodic(F.p, F.Ap, G, S.order, sc, c->stream));
-            HIP_TRY(launch_axpbypgz(shift, F.p, 1.0, F.Ap, 0.0, nullptr, n, c->stream));   // (A + s) p
-            if ((rc = scf_dot(c, F.p, F.Ap, 1, nullptr))) return rc;
-            HIP_TRY(launch_cg_xr(y, F.r, F.p, F.Ap, F.s, n, c->stream));
-            if ((rc = scf_dot(c, F.r, F.r, 2, nullptr))) return rc;
-            HIP_TRY(launch_cg_p(F.p, F.r, F.s, n, c->stream));
+            HIP_TRY(launch_cg_step(y, F.r, F.p, F.Ap, F.s + 2 * (k & 1), F.s + 2 - 2 * (k & 1), shift, G, S.order, sc, F.part,
+                                   kRedBlocks, c->stream));
         }
         HIP_TRY(hipMemcpyAsync(&rr, F.s, sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1738,11 +1723,8 @@ static int enqueue_poisson(sq_ctx *c, const double *f, double tol, bool eager)
     const int *sk = &ctl->pdone;
     auto block = [&]() -> int {
         for (int k = 0; k < 4; k++) {
-            HIP_TRY(launch_lap_periodic(F.p, F.Ap, G, S.order, sc, st, sk));
-            HIP_TRY(launch_dot(F.p, F.Ap, n, 1.0, F.part, kRedBlocks, F.s + 1, st, sk));
-            HIP_TRY(launch_cg_xr(F.phi, F.r, F.p, F.Ap, F.s, n, st, sk));
-            HIP_TRY(launch_dot(F.r, F.r, n, 1.0, F.part, kRedBlocks, F.s + 2, st, sk));
-            HIP_TRY(launch_cg_p(F.p, F.r, F.s, n, st, sk));
+            HIP_TRY(launch_cg_step(F.phi, F.r, F.p, F.Ap, F.s + 2 * (k & 1), F.s + 2 - 2 * (k & 1), 0.0, G, S.order, sc, F.part,
+                                   kRedBlocks, st, sk));
         }
         HIP_TRY(launch_cg_check(F.s, &ctl->pstop, &ctl->pdone, &ctl->piters, 20000, st));
         return SQ_OK;
@@ -1775,12 +1757,8 @@ static int enqueue_kerker(sq_ctx *c, const double *u, double *y, double k0, bool
     const int *sk = &ctl->kdone;
     auto block = [&]() -> int {
         for (int k = 0; k < 4; k++) {
-            HIP_TRY(launch_lap_periodic(F.p, F.Ap, G, S.order, sc, st, sk));
-            HIP_TRY(launch_axpbypgz(shift, F.p, 1.0, F.Ap, 0.0, nullptr, n, st, sk));
-            HIP_TRY(launch_dot(F.p, F.Ap, n, 1.0, F.part, kRedBlocks, F.s + 1, st, sk));
-            HIP_TRY(launch_cg_xr(y, F.r, F.p, F.Ap, F.s, n, st, sk));
-            HIP_TRY(launch_dot(F.r, F.r, n, 1.0, F.part, kRedBlocks, F.s + 2, st, sk));
-            HIP_TRY(launch_cg_p(F.p, F.r, F.s, n, st, sk));
+            HIP_TRY(launch_cg_step(y, F.r, F.p, F.Ap, F.s + 2 * (k & 1), F.s + 2 - 2 * (k & 1), shift, G, S.order, sc, F.part,
+                                   kRedBlocks, st, sk));
         }
         HIP_TRY(launch_cg_check(F.s, &ctl->kstop, &ctl->kdone, &ctl->kiters, 2000, st));
         return SQ_OK;
@@ -1835,19 +1813,10 @@ static int enqueue_fermi_density(sq_ctx *c, double *rho_out)
     hipStream_t st = c->stream;
     ScfCtl *ctl = c->scf.ctl;
     HIP_TRY(launch_lam_range(c->lmin, c->lmax, nn, c->out, st));
-    HIP_TRY(launch_bis_begin(c->out, ctl, st));
-    HIP_TRY(launch_occupation_partial_dev(c->lam, c->w, nq, beta, &ctl->lo, nullptr, c->partial, kRedBlocks, st));
-    HIP_TRY(launch_bis_store(c->partial, kRedBlocks, &ctl->glo, st));
-    HIP_TRY(launch_occupation_partial_dev(c->lam, c->w, nq, beta, &ctl->hi, nullptr, c->partial, kRedBlocks, st));
-    HIP_TRY(launch_bis_store(c->partial, kRedBlocks, &ctl->ghi, st));
-    HIP_TRY(launch_bis_first(ctl, nelec, st));
-    for (int k = 0; k < 200; k++) {
-        HIP_TRY(launch_occupation_partial_dev(c->lam, c->w, nq, beta, &ctl->mid, &ctl->fdone, c->partial, kRedBlocks, st));
-        HIP_TRY(launch_bis_step(c->partial, kRedBlocks, ctl, nelec, st));
-    }
-    HIP_TRY(launch_bis_end(ctl, st));
-    HIP_TRY(launch_density_energy_dev(c->lam, c->w, nn, S.nqp, beta, &ctl->lf, 2.0 / S.dV, rho_out, c->partial,
-                                      c->partial2, kRedBlocks, c->out, st));
+    for (int k = -2; k <= 200; k++)
+        HIP_TRY(launch_fermi_count(c->lam, c->w, nq, beta, nelec, c->out, k, c->bis, c->partial, st));
+    HIP_TRY(launch_bis_end(c->bis, ctl, st));   // count 200 leaves its state in slot 0
+    HIP_TRY(launch_density_energy(c->lam, c->w, nn, S.nqp, beta, &ctl->lf, 2.0 / S.dV, rho_out, c->partial, c->out, st));
     return SQ_OK;
 }
 

@@ -69,6 +69,38 @@ __device__ __forceinline__ CSum wave_csum(CSum v)
     return v;
 }
 
+// The sum of partial[0..n) in index order, to every thread of the block.  The
+// partials come to LDS together and from there a batch ahead of the chain of
+// additions: 512 take 3 us, where one thread that adds them from memory takes 20-30.
+constexpr int kSumBatch = 32;
+constexpr int ordered_lds(int n) { return (n + kSumBatch - 1) / kSumBatch * kSumBatch + 2; }   // doubles at sm
+__device__ __forceinline__ double ordered_total(const double *partial, int n, double *sm)
+{
+    const int padded = ordered_lds(n) - 2;   // zeros after the last: they leave a sum that began at +0 as it is
+    for (int k = threadIdx.x; k < padded; k += blockDim.x) sm[k] = k < n ? partial[k] : 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0, v[kSumBatch], u[kSumBatch];
+#pragma unroll
+        for (int i = 0; i < kSumBatch; i++) v[i] = sm[i];
+        for (int k = kSumBatch; k < padded; k += kSumBatch) {
+#pragma unroll
+            for (int i = 0; i < kSumBatch; i++) u[i] = sm[k + i];
+#pragma unroll
+            for (int i = 0; i < kSumBatch; i++) s += v[i];
+#pragma unroll
+            for (int i = 0; i < kSumBatch; i++) v[i] = u[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kSumBatch; i++) s += v[i];
+        sm[padded] = s;
+    }
+    __syncthreads();
+    const double s = sm[padded];
+    __syncthreads();
+    return s;
+}
+
 // Block-wide deterministic sum of one double per thread (fixed tree).
 template <int NW = kWaves>
 __device__ double block_sum(double v, double *red)

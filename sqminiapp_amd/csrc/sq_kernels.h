@@ -96,18 +96,21 @@ void *noalloc_scratch(int device);
 size_t noalloc_ql_bytes(int n, long count);
 hipError_t launch_ql_noalloc(void *ws, const double *a, const double *b, int n, long count, double *lam, double *w,
                              double *lmin, double *lmax, long long **first_bad, hipStream_t st);
-hipError_t launch_occupation(const double *lam, const double *w, long nq, double beta, double lf, double *partial,
-                             int nblocks, double *out, hipStream_t st);
-hipError_t launch_density_energy(const double *lam, const double *w, long n_nodes, int nqp, double beta, double lf,
-                                 double two_over_dv, double *rho, double *part_e, double *part_s, int nblocks,
-                                 double *out2, hipStream_t st);
+// Fermi bisection: the state after a count
+constexpr int kRedBlocksDev = 512;
+struct BisState {
+    double lo, hi, mid, lf;      // bracket, midpoint to count at, level if it stopped here
+    int done, bad, count;        // stopped; level not bracketed; halvings
+};
+// One count (sq_kernels.hip); counts -2, -1, 0, 1, ... in order on one stream.  After
+// count k the state is state[k & 1].  state: 2, partial: 3 * kRedBlocksDev doubles.
+hipError_t launch_fermi_count(const double *lam, const double *w, long nq, double beta, double nelec, const double *range,
+                              int count, BisState *state, double *partial, hipStream_t st);
+// rho (may be null), and out2 = {E_band, -TS} at the Fermi level *lf_dev; partial: 2 * kRedBlocksDev doubles
+hipError_t launch_density_energy(const double *lam, const double *w, long n_nodes, int nqp, double beta,
+                                 const double *lf_dev, double two_over_dv, double *rho, double *partial, double *out2,
+                                 hipStream_t st);
 hipError_t launch_lam_range(const double *lmin, const double *lmax, long n, double *out, hipStream_t st);
-// the same with the Fermi level read from device memory (and a skip flag)
-hipError_t launch_occupation_partial_dev(const double *lam, const double *w, long nq, double beta, const double *lf_dev,
-                                         const int *skip, double *partial, int nblocks, hipStream_t st);
-hipError_t launch_density_energy_dev(const double *lam, const double *w, long n_nodes, int nqp, double beta,
-                                     const double *lf_dev, double two_over_dv, double *rho, double *part_e, double *part_s,
-                                     int nblocks, double *out2, hipStream_t st);
 
 // ---- forces (sq_forces.hip)
 // coef[r][k] = (f(T) e_1)_k for node ids[r]'s tridiagonal (a, b at id * stride,
@@ -169,9 +172,15 @@ hipError_t launch_dot(const double *a, const double *b, long n, double scale, do
                       hipStream_t st, const int *skip = nullptr);
 hipError_t launch_axpbypgz(double alpha, const double *x, double beta, double *y, double gamma, const double *z, long n,
                            hipStream_t st, const int *skip = nullptr);
-hipError_t launch_cg_xr(double *x, double *r, const double *p, const double *Ap, const double *s, long n, hipStream_t st,
-                        const int *skip = nullptr);
-hipError_t launch_cg_p(double *p, const double *r, double *s, long n, hipStream_t st, const int *skip = nullptr);
+// One conjugate-gradient step in three launches.  The dot products' block
+// partials are summed, in block order, by the launch that needs them.
+//   Ap = A p (+ shift p when shift > 0), part <- <p, Ap>
+//   x += (rr / pAp) p, r -= (rr / pAp) Ap, part + nblocks <- <r, r>
+//   p = r + (rr_new / rr) p, rr_new -> s_new
+// rr sits at s_cur before the step and at s_new (another place) after it.
+hipError_t launch_cg_step(double *x, double *r, double *p, double *Ap, const double *s_cur, double *s_new, double shift,
+                          const int G[3], int order, const StencilCoeffs &c, double *part, int nblocks, hipStream_t st,
+                          const int *skip = nullptr);
 // m_dev (device int, may be null) replaces m
 hipError_t launch_pulay_update(const double *x, const double *f, const double *dX, const double *dF, const double *g, int m,
                                double beta, long n, double *xn, hipStream_t st, const int *m_dev = nullptr,
@@ -183,11 +192,11 @@ hipError_t launch_pulay_split(const double *x, const double *f, const double *dX
 constexpr int kMaxHist = 16;   // Pulay history limit of the device solve
 struct ScfCtl {
     double pstop, kstop;                 // CG thresholds: Poisson, Kerker
-    double lo, hi, mid, lf, glo, ghi;    // Fermi bisection
+    double lf;                           // Fermi level
     double gram[kMaxHist * kMaxHist], rhs[kMaxHist], g[kMaxHist];   // Pulay Gram system, coefficients
     int pdone, piters, pfail;            // Poisson CG: stopped, iterations, not converged
     int kdone, kiters, kfail;            // Kerker CG
-    int fdone, fbad, fcount;             // bisection: stopped, level not bracketed, counts
+    int fbad;                            // bisection: level not bracketed
     int it, head, nhist, mu;             // SCF iteration; Pulay history slot, length, coefficients used
     int conv, nopush, pulay, bad;        // SCF stopped; no history push; Pulay step; first bad node (-1)
     int gskip[kMaxHist];                 // Gram row a not needed this step
@@ -201,11 +210,7 @@ hipError_t launch_axpb_mean(double alpha, const double *x, double *y, double msc
 hipError_t launch_copy(double *dst, const double *src, long n, const int *skip, hipStream_t st);
 hipError_t launch_zero(double *y, long n, const int *skip, hipStream_t st);
 hipError_t launch_zero_int(int *y, int n, hipStream_t st);
-hipError_t launch_bis_begin(const double *range, ScfCtl *c, hipStream_t st);
-hipError_t launch_bis_store(const double *partial, int nblocks, double *out, hipStream_t st);
-hipError_t launch_bis_first(ScfCtl *c, double nelec, hipStream_t st);
-hipError_t launch_bis_step(const double *partial, int nblocks, ScfCtl *c, double nelec, hipStream_t st);
-hipError_t launch_bis_end(ScfCtl *c, hipStream_t st);
+hipError_t launch_bis_end(const BisState *b, ScfCtl *c, hipStream_t st);
 hipError_t launch_status_any(const int *status, long n, ScfCtl *c, hipStream_t st);
 hipError_t launch_conv(const double *s, ScfCtl *c, double tol, hipStream_t st);
 hipError_t launch_hist_push(const double *x, const double *xp, const double *f, const double *fp, double *dX, double *dF,

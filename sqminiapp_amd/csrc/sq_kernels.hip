@@ -403,14 +403,10 @@ __device__ __forceinline__ double fermi_ent(double x)  // f ln f + (1-f) ln(1-f)
 
 constexpr int kRedThreads = 256;
 
-// partial[block] = sum over the block's chunk of w * f(beta (lam - lf))
-__global__ void __launch_bounds__(kRedThreads) occupation_partial(const double *lam, const double *w, long nq, double beta,
-                                                                  double lf, double *partial, const double *lf_dev,
-                                                                  const int *skip)
+// A block's partial of sum w f(beta (lam - lf)) over its chunk
+__device__ __forceinline__ void occupation_block(const double *lam, const double *w, long nq, double beta, double lf,
+                                                 double *partial, double *red)
 {
-    if (skip && *skip) return;
-    if (lf_dev) lf = *lf_dev;
-    __shared__ double red[kRedThreads / 64];
     const long chunk = (nq + gridDim.x - 1) / gridDim.x;
     const long q0 = blockIdx.x * chunk, q1 = min(nq, q0 + chunk);
     double s = 0.0;
@@ -425,37 +421,102 @@ __global__ void __launch_bounds__(kRedThreads) occupation_partial(const double *
     }
 }
 
-// sum of partials in index order -> out[0]
-__global__ void ordered_sum(const double *partial, int n, double scale, double *out)
+// One electron count of the Fermi bisection, N(lf) = 2 sum w f, on [lambda_min
+// - 1, lambda_max + 1] to 1e-14 (relative) in at most 200 halvings.  A launch
+// first takes the decision that the last count calls for -- every block for
+// itself, from the last launch's partials and state, so no launch is spent on
+// it -- and then counts at the new midpoint.  Count k leaves its state at state[k
+// & 1] and its partials in the (k + 2) % 3-th of three places: no block of a launch
+// writes what another still reads.  count: -2 at the lower end, -1 at the upper
+// end, then 0 (brackets, first midpoint), 1, ...  A halving takes 5 us; the count,
+// its sum and a look by the host took 60, on the device 16 in two launches.
+__global__ void __launch_bounds__(kRedThreads) fermi_count(const double *lam, const double *w, long nq, double beta,
+                                                           double nelec, const double *range, int count, BisState *state,
+                                                           double *partial)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int k = 0; k < n; k++) s += partial[k];
-        out[0] = scale * s;
+    __shared__ double red[kRedThreads / 64], sm[ordered_lds(kRedBlocksDev)];
+    const int nb = gridDim.x;
+    double *const mine = partial + (count + 2) % 3 * nb;
+    if (count < 0) {
+        occupation_block(lam, w, nq, beta, count == -2 ? range[0] - 1.0 : range[1] + 1.0, mine, red);
+        return;
     }
+    BisState b;
+    if (count == 0) {
+        b.lo = range[0] - 1.0;
+        b.hi = range[1] + 1.0;
+        b.mid = 0.0;
+        b.done = b.bad = b.count = 0;
+        const double glo = 2.0 * ordered_total(partial, nb, sm);
+        const double ghi = 2.0 * ordered_total(partial + nb, nb, sm);
+        if (glo - nelec > 0 || ghi - nelec < 0) b.bad = b.done = 1;
+    } else {
+        b = state[(count - 1) & 1];
+        if (!b.done) {
+            const double g = 2.0 * ordered_total(partial + (count + 1) % 3 * nb, nb, sm);
+            if (g - nelec > 0) b.hi = b.mid;
+            else b.lo = b.mid;
+            if (++b.count >= 200) b.done = 1;
+        }
+    }
+    if (!b.done) {
+        b.mid = 0.5 * (b.lo + b.hi);
+        if (b.hi - b.lo <= 1e-14 * (fabs(b.mid) > 1.0 ? fabs(b.mid) : 1.0)) b.done = 1;
+    }
+    b.lf = 0.5 * (b.lo + b.hi);
+    if (threadIdx.x == 0 && blockIdx.x == 0) state[count & 1] = b;
+    if (!b.done) occupation_block(lam, w, nq, beta, b.mid, mine, red);
 }
 
-// per node: rho = (2/dV) sum_i w f; partials of sum w lam f and sum w S(f)
-__global__ void __launch_bounds__(kRedThreads) density_energy(const double *lam, const double *w, long n_nodes, int nqp,
-                                                              double beta, double lf, double two_over_dv, double *rho,
-                                                              double *part_e, double *part_s, const double *lf_dev)
+// sum of partials in index order -> out[0]
+__global__ void __launch_bounds__(64) ordered_sum(const double *partial, int n, double scale, double *out)
 {
-    if (lf_dev) lf = *lf_dev;
+    __shared__ double sm[ordered_lds(kRedBlocksDev)];
+    const double s = ordered_total(partial, n, sm);
+    if (threadIdx.x == 0) out[0] = scale * s;
+}
+
+// per node: rho = (2/dV) sum_i w f; partials of sum w lam f and sum w S(f).  The
+// block's threads form the terms of its nodes' rules together, a node's own
+// thread adds them in order: one thread a node, as before, left 8 of 256 busy
+// with the exponentials (3840 nodes: 12 us, and 90 before).
+__global__ void __launch_bounds__(kRedThreads) density_energy(const double *lam, const double *w, long n_nodes, int nqp,
+                                                              double beta, const double *lf_dev, double two_over_dv,
+                                                              double *rho, double *part_e, double *part_s)
+{
+    constexpr int kTerms = 1024;
+    __shared__ double tr[kTerms], te[kTerms], ts[kTerms];
     __shared__ double re[kRedThreads / 64], rs[kRedThreads / 64];
+    const double lf = *lf_dev;
     const long chunk = (n_nodes + gridDim.x - 1) / gridDim.x;
     const long p0 = blockIdx.x * chunk, p1 = min(n_nodes, p0 + chunk);
     double se = 0.0, ss = 0.0;
-    for (long p = p0 + threadIdx.x; p < p1; p += blockDim.x) {
+    for (long base = p0; base < p1; base += blockDim.x) {
+        const int rows = (int)min((long)blockDim.x, p1 - base), width = min(nqp, kTerms / rows);
+        const bool mine = (int)threadIdx.x < rows;
         double sr = 0.0;
-        for (int i = 0; i < nqp; i++) {
-            const long q = p * nqp + i;
-            const double x = beta * (lam[q] - lf);
-            const double f = fermi_occ(x);
-            sr += w[q] * f;
-            se += w[q] * lam[q] * f;
-            ss += w[q] * fermi_ent(x);
+        for (int i0 = 0; i0 < nqp; i0 += width) {
+            const int cols = min(width, nqp - i0);
+            for (int k = threadIdx.x; k < rows * cols; k += blockDim.x) {
+                const int row = k / cols;
+                const long q = (base + row) * nqp + i0 + (k - row * cols);
+                const double x = beta * (lam[q] - lf);
+                const double f = fermi_occ(x);
+                tr[k] = w[q] * f;
+                te[k] = w[q] * lam[q] * f;
+                ts[k] = w[q] * fermi_ent(x);
+            }
+            __syncthreads();
+            if (mine)
+                for (int i = 0; i < cols; i++) {
+                    const int k = threadIdx.x * cols + i;
+                    sr += tr[k];
+                    se += te[k];
+                    ss += ts[k];
+                }
+            __syncthreads();
         }
-        if (rho) rho[p] = two_over_dv * sr;
+        if (rho && mine) rho[base + threadIdx.x] = two_over_dv * sr;
     }
     se = wave_sum(se);
     ss = wave_sum(ss);
@@ -470,16 +531,22 @@ __global__ void __launch_bounds__(kRedThreads) density_energy(const double *lam,
 }
 
 // min/max of lambda over all nodes (bracket of the Fermi level)
-__global__ void lam_range(const double *lmin, const double *lmax, long n, double *out)
+__global__ void __launch_bounds__(1024) lam_range(const double *lmin, const double *lmax, long n, double *out)
 {
-    __shared__ double smin[kRedThreads], smax[kRedThreads];
+    __shared__ double smin[16], smax[16];
     double a = 1e300, b = -1e300;
     for (long p = threadIdx.x; p < n; p += blockDim.x) { a = fmin(a, lmin[p]); b = fmax(b, lmax[p]); }
-    smin[threadIdx.x] = a;
-    smax[threadIdx.x] = b;
+    for (int off = 32; off > 0; off >>= 1) {
+        a = fmin(a, __shfl_xor(a, off, 64));
+        b = fmax(b, __shfl_xor(b, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        smin[threadIdx.x >> 6] = a;
+        smax[threadIdx.x >> 6] = b;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int k = 1; k < (int)blockDim.x; k++) { a = fmin(a, smin[k]); b = fmax(b, smax[k]); }
+        for (int k = 1; k < 16; k++) { a = fmin(a, smin[k]); b = fmax(b, smax[k]); }
         out[0] = a;
         out[1] = b;
     }
@@ -547,48 +614,29 @@ hipError_t launch_ql(const double *a, const double *b, int n, int stride, long c
     return hipGetLastError();
 }
 
-hipError_t launch_occupation(const double *lam, const double *w, long nq, double beta, double lf, double *partial,
-                             int nblocks, double *out, hipStream_t st)
+hipError_t launch_fermi_count(const double *lam, const double *w, long nq, double beta, double nelec, const double *range,
+                              int count, BisState *state, double *partial, hipStream_t st)
 {
-    hipLaunchKernelGGL(occupation_partial, dim3(nblocks), dim3(kRedThreads), 0, st, lam, w, nq, beta, lf, partial,
-                       (const double *)nullptr, (const int *)nullptr);
-    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, partial, nblocks, 2.0, out);
+    hipLaunchKernelGGL(fermi_count, dim3(kRedBlocksDev), dim3(kRedThreads), 0, st, lam, w, nq, beta, nelec, range, count,
+                       state, partial);
     return hipGetLastError();
 }
 
-hipError_t launch_density_energy(const double *lam, const double *w, long n_nodes, int nqp, double beta, double lf,
-                                 double two_over_dv, double *rho, double *part_e, double *part_s, int nblocks,
-                                 double *out2, hipStream_t st)
+hipError_t launch_density_energy(const double *lam, const double *w, long n_nodes, int nqp, double beta,
+                                 const double *lf_dev, double two_over_dv, double *rho, double *partial, double *out2,
+                                 hipStream_t st)
 {
-    hipLaunchKernelGGL(density_energy, dim3(nblocks), dim3(kRedThreads), 0, st, lam, w, n_nodes, nqp, beta, lf,
-                       two_over_dv, rho, part_e, part_s, (const double *)nullptr);
-    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_e, nblocks, 2.0, out2);
-    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_s, nblocks, 2.0 / beta, out2 + 1);
-    return hipGetLastError();
-}
-
-hipError_t launch_occupation_partial_dev(const double *lam, const double *w, long nq, double beta, const double *lf_dev,
-                                         const int *skip, double *partial, int nblocks, hipStream_t st)
-{
-    hipLaunchKernelGGL(occupation_partial, dim3(nblocks), dim3(kRedThreads), 0, st, lam, w, nq, beta, 0.0, partial, lf_dev,
-                       skip);
-    return hipGetLastError();
-}
-
-hipError_t launch_density_energy_dev(const double *lam, const double *w, long n_nodes, int nqp, double beta,
-                                     const double *lf_dev, double two_over_dv, double *rho, double *part_e, double *part_s,
-                                     int nblocks, double *out2, hipStream_t st)
-{
-    hipLaunchKernelGGL(density_energy, dim3(nblocks), dim3(kRedThreads), 0, st, lam, w, n_nodes, nqp, beta, 0.0,
-                       two_over_dv, rho, part_e, part_s, lf_dev);
-    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_e, nblocks, 2.0, out2);
-    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_s, nblocks, 2.0 / beta, out2 + 1);
+    double *const part_e = partial, *const part_s = partial + kRedBlocksDev;
+    hipLaunchKernelGGL(density_energy, dim3(kRedBlocksDev), dim3(kRedThreads), 0, st, lam, w, n_nodes, nqp, beta, lf_dev,
+                       two_over_dv, rho, part_e, part_s);
+    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_e, kRedBlocksDev, 2.0, out2);
+    hipLaunchKernelGGL(ordered_sum, dim3(1), dim3(64), 0, st, part_s, kRedBlocksDev, 2.0 / beta, out2 + 1);
     return hipGetLastError();
 }
 
 hipError_t launch_lam_range(const double *lmin, const double *lmax, long n, double *out, hipStream_t st)
 {
-    hipLaunchKernelGGL(lam_range, dim3(1), dim3(kRedThreads), 0, st, lmin, lmax, n, out);
+    hipLaunchKernelGGL(lam_range, dim3(1), dim3(1024), 0, st, lmin, lmax, n, out);
     return hipGetLastError();
 }
 

@@ -7,7 +7,7 @@
 // partials in block order, so results do not depend on scheduling.
 #include <algorithm>
 
-#include "sq_kernels.h"
+#include "sq_device_common.h"
 
 namespace sqamd {
 
@@ -55,28 +55,41 @@ __global__ void __launch_bounds__(kT) xc_lda_pw(const double *__restrict__ rho, 
     }
 }
 
-// y = -(1/2) Lap_h x on the periodic cell G0 x G1 x G2 (the reference's
-// Poisson operator, Create_Laplacian, lsdft_initObjs.cc:309-388, on a periodic
-// DMDA): y = (c0x+c0y+c0z) x + sum_a c_a (x(-a) + x(+a)) per axis.
+// -(1/2) Lap_h x at point (i, j, k) of the periodic cell G0 x G1 x G2 (the
+// reference's Poisson operator, Create_Laplacian, lsdft_initObjs.cc:309-388, on a
+// periodic DMDA): (c0x+c0y+c0z) x + sum_a c_a (x(-a) + x(+a)) per axis.  ORDER > 0: the
+// order, its loads all in flight at once.
+template <int ORDER>
+__device__ __forceinline__ double lap_at(const double *__restrict__ x, int i, int j, int k, int G0, int G1, int G2,
+                                         int order, const StencilCoeffs &c)
+{
+    if (ORDER) order = ORDER;
+    const long row = (long)G0, plane = row * G1;
+    const double *const xi = x + k * plane + j * row, *const xj = x + k * plane + i, *const xk = x + j * row + i;
+    double s = (c.w[0][0] + c.w[1][0] + c.w[2][0]) * xi[i];
+    int im = i, ip = i, jm = j, jp = j, km = k, kp = k;
+#pragma unroll ORDER ? ORDER : 1
+    for (int a = 1; a <= order; a++) {   // the neighbours step around the cell, also one narrower than the order
+        im = (im ? im : G0) - 1;
+        ip = ip + 1 < G0 ? ip + 1 : 0;
+        jm = (jm ? jm : G1) - 1;
+        jp = jp + 1 < G1 ? jp + 1 : 0;
+        km = (km ? km : G2) - 1;
+        kp = kp + 1 < G2 ? kp + 1 : 0;
+        s += c.w[0][a] * (xi[im] + xi[ip]) + c.w[1][a] * (xj[jm * row] + xj[jp * row]) +
+             c.w[2][a] * (xk[km * plane] + xk[kp * plane]);
+    }
+    return s;
+}
+
 __global__ void __launch_bounds__(kT) lap_periodic(const double *__restrict__ x, double *__restrict__ y, int G0, int G1,
                                                     int G2, int order, StencilCoeffs c, const int *skip)
 {
     if (skip && *skip) return;
     const long n = (long)G0 * G1 * G2;
     for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(q % G0);
-        const int j = (int)((q / G0) % G1);
-        const int k = (int)(q / ((long)G0 * G1));
-        double s = (c.w[0][0] + c.w[1][0] + c.w[2][0]) * x[q];
-        for (int a = 1; a <= order; a++) {
-            const int im = ((i - a) % G0 + G0) % G0, ip = (i + a) % G0;
-            const int jm = ((j - a) % G1 + G1) % G1, jp = (j + a) % G1;
-            const int km = ((k - a) % G2 + G2) % G2, kp = (k + a) % G2;
-            const long row = ((long)k * G1 + j) * G0;
-            s += c.w[0][a] * (x[row + im] + x[row + ip]) + c.w[1][a] * (x[((long)k * G1 + jm) * G0 + i] + x[((long)k * G1 + jp) * G0 + i]) +
-                 c.w[2][a] * (x[((long)km * G1 + j) * G0 + i] + x[((long)kp * G1 + j) * G0 + i]);
-        }
-        y[q] = s;
+        const long t = q / G0;
+        y[q] = lap_at<0>(x, (int)(q - t * G0), (int)(t % G1), (int)(t / G1), G0, G1, G2, order, c);
     }
 }
 
@@ -95,15 +108,13 @@ __global__ void __launch_bounds__(kT) dot_partial(const double *__restrict__ a, 
 }
 
 // out[slot] = scale * sum of the partials, in block order.
-__global__ void sum_partials(const double *__restrict__ partial, int n, double scale, double *__restrict__ out,
-                             const int *skip)
+__global__ void __launch_bounds__(64) sum_partials(const double *__restrict__ partial, int n, double scale,
+                                                   double *__restrict__ out, const int *skip)
 {
     if (skip && *skip) return;
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int k = 0; k < n; k++) s += partial[k];
-        out[0] = scale * s;
-    }
+    extern __shared__ double sm[];
+    const double s = ordered_total(partial, n, sm);
+    if (threadIdx.x == 0) out[0] = scale * s;
 }
 
 // y = alpha x + gamma z + beta y; with z null the constant gamma is added;
@@ -119,33 +130,78 @@ __global__ void __launch_bounds__(kT) axpbypgz(double alpha, const double *x, do
     }
 }
 
-// Conjugate-gradient step with the scalars on the device: s = {rr, pAp, rr_new, ...}.
-// x += (rr/pAp) p ; r -= (rr/pAp) Ap
-__global__ void __launch_bounds__(kT) cg_xr(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
-                                            const double *__restrict__ Ap, const double *__restrict__ s, long n,
-                                            const int *skip)
+// A conjugate-gradient step (launch_cg_step).  Every dot product runs over the
+// chunks of dot_partial, in the launch that forms its vector; its partials are
+// summed by every block of the next launch, which costs 4 us there where launches of
+// their own for the sum and the scalars cost 35.  The first operands of a block's chunk
+// are on the way meanwhile.  Bound by those chains: 157248 points take 7, 8 and 8 us
+// (86 a step in seven launches), of which their 12 passes over memory are 3.
+template <int ORDER>
+__global__ void __launch_bounds__(kT) cg_ap(const double *__restrict__ p, double *__restrict__ Ap, int G0, int G1, int G2,
+                                            int order, StencilCoeffs c, double shift, long chunk,
+                                            double *__restrict__ part, const int *skip)
 {
     if (skip && *skip) return;
-    const double alpha = s[0] / s[1];
-    for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-        x[q] = fma(alpha, p[q], x[q]);
-        r[q] = fma(-alpha, Ap[q], r[q]);
+    __shared__ double sh[kT / 64];
+    const long n = (long)G0 * G1 * G2;
+    const long p0 = blockIdx.x * chunk, p1 = min(n, p0 + chunk);
+    const long row0 = p0 / G0;                                                    // the chunk's first point; its others
+    const int i0 = (int)(p0 - row0 * G0), k0 = (int)(row0 / G1), j0 = (int)(row0 - (long)k0 * G1);   // by 32-bit division
+    double s = 0.0;
+    for (long q = p0 + threadIdx.x; q < p1; q += blockDim.x) {
+        const unsigned ii = (unsigned)(q - p0) + i0, dj = ii / (unsigned)G0, jj = j0 + dj, dk = jj / (unsigned)G1;
+        double y = lap_at<ORDER>(p, ii - dj * G0, jj - dk * G1, k0 + dk, G0, G1, G2, order, c);
+        if (shift > 0.0) y = shift * p[q] + y;
+        Ap[q] = y;
+        s += p[q] * y;
     }
+    s = block_reduce(s, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// p = r + (rr_new/rr) p, then rr := rr_new
-__global__ void __launch_bounds__(kT) cg_p(double *__restrict__ p, const double *__restrict__ r, double *__restrict__ s, long n,
-                                           const int *skip)
+__global__ void __launch_bounds__(kT) cg_xr(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
+                                            const double *__restrict__ Ap, const double *__restrict__ s_cur, long n, long chunk,
+                                            const double *__restrict__ part, double *__restrict__ part_r, const int *skip)
 {
     if (skip && *skip) return;
-    const double beta = s[2] / s[0];
-    for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x)
-        p[q] = fma(beta, p[q], r[q]);
+    extern __shared__ double sm[];
+    __shared__ double sh[kT / 64];
+    const long p0 = blockIdx.x * chunk, p1 = min(n, p0 + chunk);
+    long q = p0 + threadIdx.x;
+    double xq = 0.0, rq = 0.0, pq = 0.0, aq = 0.0;
+    if (q < p1) { xq = x[q]; rq = r[q]; pq = p[q]; aq = Ap[q]; }
+    const double alpha = s_cur[0] / ordered_total(part, gridDim.x, sm);
+    double s = 0.0;
+    while (q < p1) {
+        x[q] = fma(alpha, pq, xq);
+        rq = fma(-alpha, aq, rq);
+        r[q] = rq;
+        s += rq * rq;
+        q += blockDim.x;
+        if (q < p1) { xq = x[q]; rq = r[q]; pq = p[q]; aq = Ap[q]; }
+    }
+    s = block_reduce(s, sh);
+    if (threadIdx.x == 0) part_r[blockIdx.x] = s;
 }
-__global__ void cg_roll(double *s, const int *skip)
+
+__global__ void __launch_bounds__(kT) cg_p(double *__restrict__ p, const double *__restrict__ r,
+                                           const double *__restrict__ s_cur, double *__restrict__ s_new, long n, long chunk,
+                                           const double *__restrict__ part_r, const int *skip)
 {
     if (skip && *skip) return;
-    if (threadIdx.x == 0 && blockIdx.x == 0) s[0] = s[2];
+    extern __shared__ double sm[];
+    const long p0 = blockIdx.x * chunk, p1 = min(n, p0 + chunk);
+    long q = p0 + threadIdx.x;
+    double pq = 0.0, rq = 0.0;
+    if (q < p1) { pq = p[q]; rq = r[q]; }
+    const double rr = ordered_total(part_r, gridDim.x, sm);
+    const double beta = rr / s_cur[0];
+    if (threadIdx.x == 0 && blockIdx.x == 0) s_new[0] = rr;
+    while (q < p1) {
+        p[q] = fma(beta, pq, rq);
+        q += blockDim.x;
+        if (q < p1) { pq = p[q]; rq = r[q]; }
+    }
 }
 
 // Periodic Pulay update x_new = x + beta f - sum_j g_j (dX_j + beta dF_j);
@@ -222,7 +278,8 @@ hipError_t launch_dot(const double *a, const double *b, long n, double scale, do
                       hipStream_t st, const int *skip)
 {
     hipLaunchKernelGGL(dot_partial, dim3(nblocks), dim3(kT), 0, st, a, b, n, partial, skip);
-    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(64), 0, st, partial, nblocks, scale, out, skip);
+    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(64), ordered_lds(nblocks) * sizeof(double), st, partial, nblocks,
+                       scale, out, skip);
     return hipGetLastError();
 }
 
@@ -233,17 +290,19 @@ hipError_t launch_axpbypgz(double alpha, const double *x, double beta, double *y
     return hipGetLastError();
 }
 
-hipError_t launch_cg_xr(double *x, double *r, const double *p, const double *Ap, const double *s, long n, hipStream_t st,
-                        const int *skip)
+hipError_t launch_cg_step(double *x, double *r, double *p, double *Ap, const double *s_cur, double *s_new, double shift,
+                          const int G[3], int order, const StencilCoeffs &c, double *part, int nblocks, hipStream_t st,
+                          const int *skip)
 {
-    hipLaunchKernelGGL(cg_xr, grid_for(n), dim3(kT), 0, st, x, r, p, Ap, s, n, skip);
-    return hipGetLastError();
-}
-
-hipError_t launch_cg_p(double *p, const double *r, double *s, long n, hipStream_t st, const int *skip)
-{
-    hipLaunchKernelGGL(cg_p, grid_for(n), dim3(kT), 0, st, p, r, s, n, skip);
-    hipLaunchKernelGGL(cg_roll, dim3(1), dim3(64), 0, st, s, skip);
+    const long n = (long)G[0] * G[1] * G[2];
+    const long chunk = (n + nblocks - 1) / nblocks;
+    const size_t lds = ordered_lds(nblocks) * sizeof(double);
+    const dim3 g(nblocks), b(kT);
+    if (order == 6)   // the order of every deck here; with the loop over it 8.6 us, not 7
+        hipLaunchKernelGGL(cg_ap<6>, g, b, 0, st, p, Ap, G[0], G[1], G[2], order, c, shift, chunk, part, skip);
+    else hipLaunchKernelGGL(cg_ap<0>, g, b, 0, st, p, Ap, G[0], G[1], G[2], order, c, shift, chunk, part, skip);
+    hipLaunchKernelGGL(cg_xr, g, b, lds, st, x, r, p, Ap, s_cur, n, chunk, part, part + nblocks, skip);
+    hipLaunchKernelGGL(cg_p, g, b, lds, st, p, r, s_cur, s_new, n, chunk, part + nblocks, skip);
     return hipGetLastError();
 }
 

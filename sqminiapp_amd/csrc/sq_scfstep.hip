@@ -68,60 +68,11 @@ __global__ void k_zero_int(int *y, int n)
     for (int q = threadIdx.x; q < n; q += blockDim.x) y[q] = 0;
 }
 
-// ---- Fermi level: bisection on [lambda_min - 1, lambda_max + 1] to 1e-14
-// (relative), at most 200 occupation counts (the host loop it replaces)
-__global__ void k_bis_begin(const double *range, ScfCtl *c)
+__global__ void k_bis_end(const BisState *b, ScfCtl *c)
 {
     if (threadIdx.x || blockIdx.x) return;
-    c->lo = range[0] - 1.0;
-    c->hi = range[1] + 1.0;
-    c->fdone = 0;
-    c->fbad = 0;
-    c->fcount = 0;
-}
-
-// N(lf) = 2 sum of the occupation partials, in block order
-__global__ void k_bis_store(const double *partial, int nblocks, double *out)
-{
-    if (threadIdx.x || blockIdx.x) return;
-    double s = 0.0;
-    for (int k = 0; k < nblocks; k++) s += partial[k];
-    *out = 2.0 * s;
-}
-
-__device__ __forceinline__ void bis_mid(ScfCtl *c)
-{
-    c->mid = 0.5 * (c->lo + c->hi);
-    if (c->hi - c->lo <= 1e-14 * (fabs(c->mid) > 1.0 ? fabs(c->mid) : 1.0)) c->fdone = 1;
-}
-
-__global__ void k_bis_first(ScfCtl *c, double nelec)
-{
-    if (threadIdx.x || blockIdx.x) return;
-    if (c->glo - nelec > 0 || c->ghi - nelec < 0) {
-        c->fbad = 1;
-        c->fdone = 1;
-        return;
-    }
-    bis_mid(c);
-}
-
-__global__ void k_bis_step(const double *partial, int nblocks, ScfCtl *c, double nelec)
-{
-    if (threadIdx.x || blockIdx.x || c->fdone) return;
-    double s = 0.0;
-    for (int k = 0; k < nblocks; k++) s += partial[k];
-    const double g = 2.0 * s;
-    if (g - nelec > 0) c->hi = c->mid;
-    else c->lo = c->mid;
-    if (++c->fcount >= 200) { c->fdone = 1; return; }
-    bis_mid(c);
-}
-
-__global__ void k_bis_end(ScfCtl *c)
-{
-    if (threadIdx.x || blockIdx.x) return;
-    c->lf = 0.5 * (c->lo + c->hi);
+    c->lf = b->lf;
+    c->fbad = b->bad;
 }
 
 // first node (lowest index) whose status is not 0, or -1
@@ -263,29 +214,9 @@ hipError_t launch_zero_int(int *y, int n, hipStream_t st)
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, y, n);
     return hipGetLastError();
 }
-hipError_t launch_bis_begin(const double *range, ScfCtl *c, hipStream_t st)
+hipError_t launch_bis_end(const BisState *b, ScfCtl *c, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_bis_begin, dim3(1), dim3(64), 0, st, range, c);
-    return hipGetLastError();
-}
-hipError_t launch_bis_store(const double *partial, int nblocks, double *out, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_bis_store, dim3(1), dim3(64), 0, st, partial, nblocks, out);
-    return hipGetLastError();
-}
-hipError_t launch_bis_first(ScfCtl *c, double nelec, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_bis_first, dim3(1), dim3(64), 0, st, c, nelec);
-    return hipGetLastError();
-}
-hipError_t launch_bis_step(const double *partial, int nblocks, ScfCtl *c, double nelec, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_bis_step, dim3(1), dim3(64), 0, st, partial, nblocks, c, nelec);
-    return hipGetLastError();
-}
-hipError_t launch_bis_end(ScfCtl *c, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_bis_end, dim3(1), dim3(64), 0, st, c);
+    hipLaunchKernelGGL(k_bis_end, dim3(1), dim3(64), 0, st, b, c);
     return hipGetLastError();
 }
 hipError_t launch_status_any(const int *status, long n, ScfCtl *c, hipStream_t st)
