@@ -11,6 +11,7 @@
 #include <cstring>
 #include <string>
 #include <functional>
+#include <mutex>
 #include <vector>
 
 #include "../../include/sq_amd.h"
@@ -2325,6 +2326,10 @@ struct sq_mlp {
     std::vector<float> mean, rstd;
     double tscale = 1.0;
     std::vector<float> X, T;
+    // device workspace of the last pass, kept for the next (at most kMlpKeep bytes)
+    std::mutex ws_lock;
+    char *ws = nullptr;
+    size_t ws_bytes = 0;
 };
 
 namespace {
@@ -2338,6 +2343,43 @@ struct DevBufs {
         HIP_TRY(hipMalloc((void **)dst, std::max<size_t>(n, 1) * sizeof(T)));
         p.push_back(*dst);
         return SQ_OK;
+    }
+};
+
+// Pieces of a model's workspace, each 256-byte aligned, while its lock is held.  It
+// grows to what a pass needs and stays, up to kMlpKeep, until the model is destroyed:
+// an allocation and a release of each piece cost a call more than its kernels.
+constexpr size_t kMlpKeep = 256u << 20;
+struct MlpSpace {
+    sq_mlp *m;
+    std::lock_guard<std::mutex> hold;
+    size_t used = 0;
+    explicit MlpSpace(sq_mlp *m_) : m(m_), hold(m_->ws_lock) {}
+    ~MlpSpace()
+    {
+        if (m->ws_bytes <= kMlpKeep) return;
+        (void)hipFree(m->ws);
+        m->ws = nullptr;
+        m->ws_bytes = 0;
+    }
+    static size_t piece(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    int reserve(size_t bytes)
+    {
+        used = 0;
+        if (bytes <= m->ws_bytes) return SQ_OK;
+        if (m->ws) (void)hipFree(m->ws);
+        m->ws = nullptr;
+        m->ws_bytes = 0;
+        HIP_TRY(hipMalloc((void **)&m->ws, bytes));
+        m->ws_bytes = bytes;
+        return SQ_OK;
+    }
+    template <typename T>
+    T *get(size_t n)
+    {
+        T *const p = (T *)(m->ws + used);
+        used += piece(n * sizeof(T));
+        return p;
     }
 };
 
@@ -2417,7 +2459,7 @@ int sq_mlp_create(int device, unsigned seed, sq_mlp **out)
     else if (hipMalloc((void **)&m->p, m->np * sizeof(float)) != hipSuccess ||
              hipMalloc((void **)&m->m, m->np * sizeof(float)) != hipSuccess ||
              hipMalloc((void **)&m->v, m->np * sizeof(float)) != hipSuccess ||
-             hipMalloc((void **)&m->g, m->np * sizeof(double)) != hipSuccess)
+             hipMalloc((void **)&m->g, (m->np + 1) * sizeof(double)) != hipSuccess)
         rc = set_err(SQ_ERR_ALLOC, "network buffers");
     else if (hipMemcpy(m->p, p.data(), m->np * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
              hipMemset(m->m, 0, m->np * sizeof(float)) != hipSuccess || hipMemset(m->v, 0, m->np * sizeof(float)) != hipSuccess)
@@ -2432,7 +2474,7 @@ int sq_mlp_destroy(sq_mlp *m)
 {
     if (!m) return SQ_OK;
     (void)hipSetDevice(m->device);
-    for (void *q : {(void *)m->p, (void *)m->m, (void *)m->v, (void *)m->g})
+    for (void *q : {(void *)m->p, (void *)m->m, (void *)m->v, (void *)m->g, (void *)m->ws})
         if (q) (void)hipFree(q);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
@@ -2507,46 +2549,32 @@ int sq_mlp_add_sample_every(sq_mlp *m, sq_ctx *c, int stride)
     return SQ_OK;
 }
 
-// Activations, deltas and partial sums of one pass over N rows.
+// Rows, activations, deltas and partial sums of one pass over N rows.
 struct MlpScratch {
-    float *H1 = nullptr, *H2 = nullptr, *Z1 = nullptr, *Z2 = nullptr, *Y = nullptr, *D1 = nullptr, *D2 = nullptr,
-          *D3 = nullptr;
-    double *part = nullptr, *lsum = nullptr;
-    int nchunk = 1;
-    int alloc(DevBufs &B, long N, int H)
+    float *X, *T, *H1, *H2, *Z1, *Z2, *Y, *D1, *D2, *D3;
+    double *part;
+    int alloc(MlpSpace &W, const sq_mlp *m, long N)
     {
-        nchunk = (int)std::max<long>(1, std::min<long>(128, N / 256));
-        int rc;
-        if ((rc = B.get(&H1, N * H)) || (rc = B.get(&H2, N * H)) || (rc = B.get(&Z1, N * H)) || (rc = B.get(&Z2, N * H)) ||
-            (rc = B.get(&Y, N)) || (rc = B.get(&D1, N * H)) ||
-            (rc = B.get(&D2, N * H)) || (rc = B.get(&D3, N)) || (rc = B.get(&part, (size_t)nchunk * H * H)) ||
-            (rc = B.get(&lsum, 1)))
+        const size_t parts = (size_t)mlp_grad_chunks(N) * (m->np + 1), rows = N, wide = rows * m->H;
+        if (int rc = W.reserve(W.piece(rows * m->K * 4) + 6 * W.piece(wide * 4) + 3 * W.piece(rows * 4) + W.piece(parts * 8)))
             return rc;
+        X = W.get<float>(rows * m->K);
+        for (float **p : {&H1, &H2, &Z1, &Z2, &D1, &D2}) *p = W.get<float>(wide);
+        for (float **p : {&T, &Y, &D3}) *p = W.get<float>(rows);
+        part = W.get<double>(parts);
         return SQ_OK;
     }
 };
 
-// L and dL/dp (double) of the current parameters on normalized data already on
-// the device (X: N x K, T: N), with the activations and deltas in the scratch W
-static int mlp_loss_grad_dev(sq_mlp *m, const float *X, const float *T, long N, double *loss, const MlpScratch &W)
+// L and dL/dp (double) of the current parameters on the normalized rows W.X, W.T
+static int mlp_loss_grad_dev(sq_mlp *m, long N, double *loss, const MlpScratch &W)
 {
-    const int K = m->K, H = m->H;
-    float *H1 = W.H1, *H2 = W.H2, *Y = W.Y, *D1 = W.D1, *D2 = W.D2, *D3 = W.D3;
-    double *part = W.part, *lsum = W.lsum;
-    const int nchunk = W.nchunk;
-    HIP_TRY(launch_mlp_forward(X, N, m->p, nullptr, nullptr, H1, H2, W.Z1, W.Z2, Y, 0, m->stream));
-    HIP_TRY(launch_mlp_deltas(W.Z1, W.Z2, Y, T, N, m->p, D1, D2, D3, m->stream));
-    double *g = m->g;
-    HIP_TRY(launch_outer_sum(D1, H, X, K, N, part, nchunk, g, m->stream));                          // W1
-    HIP_TRY(launch_outer_sum(D1, H, nullptr, 1, N, part, nchunk, g + H * K, m->stream));            // b1
-    HIP_TRY(launch_outer_sum(D2, H, H1, H, N, part, nchunk, g + H * K + H, m->stream));             // W2
-    HIP_TRY(launch_outer_sum(D2, H, nullptr, 1, N, part, nchunk, g + H * K + H + H * H, m->stream)); // b2
-    HIP_TRY(launch_outer_sum(H2, H, D3, 1, N, part, nchunk, g + H * K + 2 * H + H * H, m->stream));  // w3
-    HIP_TRY(launch_outer_sum(D3, 1, nullptr, 1, N, part, nchunk, g + H * K + 3 * H + H * H, m->stream)); // b3
+    HIP_TRY(launch_mlp_forward(W.X, N, m->p, nullptr, nullptr, W.H1, W.H2, W.Z1, W.Z2, W.Y, 0, m->stream));
+    HIP_TRY(launch_mlp_deltas(W.Z1, W.Z2, W.Y, W.T, N, m->p, W.D1, W.D2, W.D3, m->stream));
+    HIP_TRY(launch_mlp_grad(W.X, W.H1, W.H2, W.D1, W.D2, W.D3, N, W.part, m->g, m->stream));
     if (loss) {
-        HIP_TRY(launch_outer_sum(D3, 1, D3, 1, N, part, nchunk, lsum, m->stream));
         double s2;
-        HIP_TRY(hipMemcpyAsync(&s2, lsum, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+        HIP_TRY(hipMemcpyAsync(&s2, m->g + m->np, sizeof(double), hipMemcpyDeviceToHost, m->stream));
         HIP_TRY(hipStreamSynchronize(m->stream));
         *loss = 0.5 * (double)N * s2;   // d3 = e / N
     }
@@ -2557,15 +2585,35 @@ int sq_mlp_loss_grad(sq_mlp *m, const float *X, const float *T, long N, double *
 {
     if (!m || !X || !T || N <= 0) return set_err(SQ_ERR_ARG, "bad argument");
     HIP_TRY(hipSetDevice(m->device));
-    DevBufs B;
-    float *dX, *dT;
-    int rc;
-    if ((rc = B.get(&dX, N * m->K)) || (rc = B.get(&dT, N))) return rc;
-    HIP_TRY(hipMemcpy(dX, X, N * m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dT, T, N * sizeof(float), hipMemcpyHostToDevice));
+    MlpSpace space(m);
     MlpScratch W;
-    if ((rc = W.alloc(B, N, m->H)) || (rc = mlp_loss_grad_dev(m, dX, dT, N, loss, W))) return rc;
+    int rc;
+    if ((rc = W.alloc(space, m, N))) return rc;
+    HIP_TRY(hipMemcpy(W.X, X, N * m->K * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(W.T, T, N * sizeof(float), hipMemcpyHostToDevice));
+    if ((rc = mlp_loss_grad_dev(m, N, loss, W))) return rc;
+    HIP_TRY(hipStreamSynchronize(m->stream));
     if (grad) HIP_TRY(hipMemcpy(grad, m->g, m->np * sizeof(double), hipMemcpyDeviceToHost));
+    return SQ_OK;
+}
+
+// Y (host) of N rows; the rows come from the host, or are already in the device's dX
+static int mlp_forward_rows(sq_mlp *m, MlpSpace &space, const float *X, const float *dX, long N, int bf16, int normalize,
+                            float *Y)
+{
+    const size_t rows = N;
+    if (!dX) {
+        if (int rc = space.reserve(space.piece(rows * m->K * 4) + space.piece(rows * 4) + 2 * space.piece(m->K * 4))) return rc;
+        float *const x = space.get<float>(rows * m->K);
+        HIP_TRY(hipMemcpy(x, X, rows * m->K * sizeof(float), hipMemcpyHostToDevice));
+        dX = x;
+    }
+    float *const dY = space.get<float>(rows), *const dmean = space.get<float>(m->K), *const drstd = space.get<float>(m->K);
+    HIP_TRY(hipMemcpy(dmean, m->mean.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(drstd, m->rstd.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(launch_mlp_forward(dX, N, m->p, normalize ? dmean : nullptr, normalize ? drstd : nullptr, nullptr, nullptr,
+                               nullptr, nullptr, dY, bf16, m->stream));
+    HIP_TRY(hipMemcpyAsync(Y, dY, N * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIP_TRY(hipStreamSynchronize(m->stream));
     return SQ_OK;
 }
@@ -2574,19 +2622,8 @@ int sq_mlp_forward(sq_mlp *m, const float *X, long N, int bf16, int normalize, f
 {
     if (!m || !X || !Y || N <= 0) return set_err(SQ_ERR_ARG, "bad argument");
     HIP_TRY(hipSetDevice(m->device));
-    DevBufs B;
-    float *dX, *dY, *dmean, *drstd;
-    int rc;
-    if ((rc = B.get(&dX, N * m->K)) || (rc = B.get(&dY, N)) || (rc = B.get(&dmean, m->K)) || (rc = B.get(&drstd, m->K)))
-        return rc;
-    HIP_TRY(hipMemcpy(dX, X, N * m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dmean, m->mean.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(drstd, m->rstd.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(launch_mlp_forward(dX, N, m->p, normalize ? dmean : nullptr, normalize ? drstd : nullptr, nullptr, nullptr,
-                               nullptr, nullptr, dY, bf16, m->stream));
-    HIP_TRY(hipMemcpyAsync(Y, dY, N * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipStreamSynchronize(m->stream));
-    return SQ_OK;
+    MlpSpace space(m);
+    return mlp_forward_rows(m, space, X, nullptr, N, bf16, normalize, Y);
 }
 
 int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
@@ -2614,20 +2651,18 @@ int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
         for (int q = 0; q < K; q++) Xn[n * K + q] = (m->X[n * K + q] - m->mean[q]) * m->rstd[q];
         Tn[n] = (float)(m->T[n] / m->tscale);
     }
-    DevBufs B;
-    float *dX, *dT;
-    int rc;
-    if ((rc = B.get(&dX, N * K)) || (rc = B.get(&dT, N))) return rc;
-    HIP_TRY(hipMemcpy(dX, Xn.data(), N * K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dT, Tn.data(), N * sizeof(float), hipMemcpyHostToDevice));
+    MlpSpace space(m);
     MlpScratch W;
-    if ((rc = W.alloc(B, N, m->H))) return rc;
+    int rc;
+    if ((rc = W.alloc(space, m, N))) return rc;
+    HIP_TRY(hipMemcpy(W.X, Xn.data(), N * K * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(W.T, Tn.data(), N * sizeof(float), hipMemcpyHostToDevice));
     for (int e = 0; e < epochs; e++) {
-        if ((rc = mlp_loss_grad_dev(m, dX, dT, N, nullptr, W))) return rc;
+        if ((rc = mlp_loss_grad_dev(m, N, nullptr, W))) return rc;
         HIP_TRY(launch_adam(m->p, m->g, m->m, m->v, m->np, (float)lr, ++m->t, m->stream));
         if ((e & 63) == 63) HIP_TRY(hipStreamSynchronize(m->stream));
     }
-    if (loss && (rc = mlp_loss_grad_dev(m, dX, dT, N, loss, W))) return rc;
+    if (loss && (rc = mlp_loss_grad_dev(m, N, loss, W))) return rc;
     HIP_TRY(hipStreamSynchronize(m->stream));
     return SQ_OK;
 }
@@ -2640,8 +2675,19 @@ int sq_mlp_guess(sq_mlp *m, sq_ctx *c, int bf16, double *rho0)
     int G[3], rc;
     if ((rc = cell_dims(c, G))) return rc;
     const long ng = (long)G[0] * G[1] * G[2];
-    std::vector<float> f(ng * kMlpK), y(ng);
-    if ((rc = sq_mlp_descriptors(c, f.data())) || (rc = sq_mlp_forward(m, f.data(), ng, bf16, 1, y.data()))) return rc;
+    std::vector<float> y(ng);
+    if (m->device == c->device) {   // the descriptors stay on the device
+        HIP_TRY(hipSetDevice(m->device));
+        MlpSpace space(m);
+        const size_t rows = ng;
+        if ((rc = space.reserve(space.piece(rows * kMlpK * 4) + space.piece(rows * 4) + 2 * space.piece(kMlpK * 4)))) return rc;
+        float *const d = space.get<float>(rows * kMlpK);
+        if ((rc = mlp_descriptors_dev(c, kMlpRf, d)) || (rc = mlp_forward_rows(m, space, nullptr, d, ng, bf16, 1, y.data())))
+            return rc;
+    } else {
+        std::vector<float> f(ng * kMlpK);
+        if ((rc = sq_mlp_descriptors(c, f.data())) || (rc = sq_mlp_forward(m, f.data(), ng, bf16, 1, y.data()))) return rc;
+    }
     std::vector<double> rat;
     double sc;
     Status st = build_atomic_density(S, rat, sc);

@@ -151,9 +151,11 @@ hipError_t launch_mlp_forward(const float *X, long N, const float *P, const floa
                               float *H2, float *Z1, float *Z2, float *Y, int bf16, hipStream_t st);
 hipError_t launch_mlp_deltas(const float *Z1, const float *Z2, const float *Y, const float *T, long N, const float *P,
                              float *D1, float *D2, float *D3, hipStream_t st);
-// out[i][j] = sum_n A[n][i] B[n][j] (B == nullptr: 1), in nchunk double partials summed in order
-hipError_t launch_outer_sum(const float *A, int a, const float *B, int b, long N, double *partial, int nchunk, double *out,
-                            hipStream_t st);
+// out: the gradient's parameter sums in the order of the parameters, then sum d3^2;
+// partial: mlp_grad_chunks(N) times as many
+int mlp_grad_chunks(long N);
+hipError_t launch_mlp_grad(const float *X, const float *H1, const float *H2, const float *D1, const float *D2,
+                           const float *D3, long N, double *partial, double *out, hipStream_t st);
 hipError_t launch_adam(float *p, const double *g, float *m, float *v, int n, float lr, int t, hipStream_t st);
 
 // FP64 -> FP32 copy of a table (sq_setup.hip)

@@ -15,9 +15,9 @@
 // the layers with FMA chains.  The layers are 32x64 and 64x64 -- far below an
 // MFMA tile's worth of reuse per point -- and the whole forward over a cell is
 // microseconds, so plain FMA is the right tool here.
-// Training (FP32, full batch): deltas per point, then the weight gradients as
-// sums over points of outer products, split over point chunks with double
-// partial sums and a fixed-order second pass (deterministic), then Adam.
+// Training (FP32, full batch): deltas per point, then all gradient sums over points
+// in one pass over point chunks, with double partial sums and a fixed-order second
+// pass (deterministic), then Adam.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -41,41 +41,82 @@ __device__ __forceinline__ float to_bf16(float x)
 
 constexpr int kRad = 16, kAng = 16, kMaxNb = 96;   // descriptor split; neighbours within rf of one point
 
+constexpr int kBrick[3] = {8, 8, 4}, kCand = 512;   // points of a block; images a block lists at a time
+
+// One point a thread, a brick of points a block.  The block first lists, in
+// order, the images that can lie within rf of its brick, then every thread
+// takes its neighbours from that list.  Bound by the exponentials of 14 neighbours and
+// their pairs: the cell of 128 atoms takes 0.31 ms; 4.6 with each point against all 3348
+// images.
 __global__ void __launch_bounds__(256) mlp_features(const double4 *__restrict__ img, int nimg, int G0, int G1, int G2,
                                                     double h0, double h1, double h2, double R0, double R1, double R2,
                                                     double rf, float *__restrict__ out, int *__restrict__ overflow)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (long)G0 * G1 * G2) return;
-    const int i = (int)(p % G0), j = (int)((p / G0) % G1), k = (int)(p / ((long)G0 * G1));
+    __shared__ double cx[kCand], cy[kCand], cz[kCand];
+    __shared__ int wcount[4];
+    const int nb0 = (G0 + kBrick[0] - 1) / kBrick[0], nb1 = (G1 + kBrick[1] - 1) / kBrick[1];
+    const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int i0 = b % nb0 * kBrick[0], j0 = b / nb0 % nb1 * kBrick[1], k0 = b / nb0 / nb1 * kBrick[2];
+    const int i = i0 + t % kBrick[0], j = j0 + t / kBrick[0] % kBrick[1], k = k0 + t / (kBrick[0] * kBrick[1]);
+    const bool inside = i < G0 && j < G1 && k < G2;
     const double x = h0 * i - R0, y = h1 * j - R1, z = h2 * k - R2;
+    // the brick's corners, and a bound that rounding cannot bring an image of a neighbour past
+    const double xa = h0 * i0 - R0, xb = h0 * min(i0 + kBrick[0], G0) - R0;
+    const double ya = h1 * j0 - R1, yb = h1 * min(j0 + kBrick[1], G1) - R1;
+    const double za = h2 * k0 - R2, zb = h2 * min(k0 + kBrick[2], G2) - R2;
+    const double reach = rf * rf * (1.0 + 1e-6);
     const double s = rf / (kRad - 1);
     double f[kRad + kAng];
 #pragma unroll
     for (int q = 0; q < kRad + kAng; q++) f[q] = 0.0;
     double nx[kMaxNb], ny[kMaxNb], nz[kMaxNb], nr[kMaxNb], nf[kMaxNb];
-    int nn = 0;
-    for (int a = 0; a < nimg; a++) {
-        const double4 X = img[a];
-        const double dx = X.x - x, dy = X.y - y, dz = X.z - z;
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        if (!(r < rf)) continue;
-        const double fc = 0.5 * (cos(M_PI * r / rf) + 1.0);
-#pragma unroll
-        for (int q = 0; q < kRad; q++) {
-            const double u = (r - q * rf / (kRad - 1)) / s;
-            f[q] += exp(-(u * u)) * fc;
+    int nn = 0, listed = 0;
+    for (int base = 0; base < nimg; base += 256) {
+        double4 X = make_double4(0.0, 0.0, 0.0, 0.0);
+        bool near = false;
+        if (base + t < nimg) {
+            X = img[base + t];
+            const double ex = fmax(0.0, fmax(xa - X.x, X.x - xb)), ey = fmax(0.0, fmax(ya - X.y, X.y - yb));
+            const double ez = fmax(0.0, fmax(za - X.z, X.z - zb));
+            near = ex * ex + ey * ey + ez * ez <= reach;
         }
-        if (nn < kMaxNb) { nx[nn] = dx; ny[nn] = dy; nz[nn] = dz; nr[nn] = r; nf[nn] = fc; }
-        nn++;
+        const unsigned long long m = __ballot(near);
+        if (lane == 0) wcount[wave] = __popcll(m);
+        __syncthreads();
+        int at = listed + __popcll(m & ((1ull << lane) - 1));
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) at += wcount[w];
+            listed += wcount[w];
+        }
+        if (near) { cx[at] = X.x; cy[at] = X.y; cz[at] = X.z; }
+        __syncthreads();
+        if (listed <= kCand - 256 && base + 256 < nimg) continue;   // room for the next 256
+        if (inside)
+            for (int a = 0; a < listed; a++) {
+                const double dx = cx[a] - x, dy = cy[a] - y, dz = cz[a] - z;
+                const double r = sqrt(dx * dx + dy * dy + dz * dz);
+                if (!(r < rf)) continue;
+                const double fc = 0.5 * (cos(M_PI * r / rf) + 1.0);
+#pragma unroll
+                for (int q = 0; q < kRad; q++) {
+                    const double u = (r - q * rf / (kRad - 1)) / s;
+                    f[q] += exp(-(u * u)) * fc;
+                }
+                if (nn < kMaxNb) { nx[nn] = dx; ny[nn] = dy; nz[nn] = dz; nr[nn] = r; nf[nn] = fc; }
+                nn++;
+            }
+        listed = 0;
+        __syncthreads();
     }
+    if (!inside) return;
     if (nn > kMaxNb) { atomicAdd(overflow, 1); nn = kMaxNb; }
     const double eta[2] = {0.005, 0.02};
-    for (int a = 0; a < nn; a++)
-        for (int b = a + 1; b < nn; b++) {
-            const double c = (nx[a] * nx[b] + ny[a] * ny[b] + nz[a] * nz[b]) / (nr[a] * nr[b]);
-            const double rr = nr[a] * nr[a] + nr[b] * nr[b];
-            const double w = nf[a] * nf[b];
+    for (int a = 0; a < nn; a++) {
+        const double ax = nx[a], ay = ny[a], az = nz[a], ar = nr[a], af = nf[a];
+        for (int c2 = a + 1; c2 < nn; c2++) {
+            const double c = (ax * nx[c2] + ay * ny[c2] + az * nz[c2]) / (ar * nr[c2]);
+            const double rr = ar * ar + nr[c2] * nr[c2];
+            const double w = af * nf[c2];
 #pragma unroll
             for (int ie = 0; ie < 2; ie++) {
                 const double e = exp(-eta[ie] * rr) * w;
@@ -90,6 +131,8 @@ __global__ void __launch_bounds__(256) mlp_features(const double4 *__restrict__ 
                 }
             }
         }
+    }
+    const long p = ((long)k * G1 + j) * G0 + i;
 #pragma unroll
     for (int q = 0; q < kRad + kAng; q++) out[p * (kRad + kAng) + q] = (float)f[q];
 }
@@ -176,25 +219,90 @@ __global__ void __launch_bounds__(256) mlp_deltas(const float *__restrict__ Z1, 
     }
 }
 
-// partial[c][i][j] = sum over the points of chunk c of A[n][i] * B[n][j] (B == nullptr: 1)
-__global__ void __launch_bounds__(256) outer_partial(const float *__restrict__ A, int a, const float *__restrict__ B, int b,
-                                                     long N, long chunk, double *__restrict__ partial)
+// The gradient sums over the points of one chunk, in double: W1 += d1 x^T, b1 +=
+// d1, W2 += d2 h1^T, b2 += d2, w3 += h2 d3, b3 += d3 and, last, sum d3^2.  A tile of
+// points' rows lies in LDS; a thread keeps a 4 x 4 piece of W2 and a 4 x 2 piece of
+// W1 in registers, so a point costs it four LDS reads and 24 multiply-adds, and a
+// column sum is one thread's.  Bound by the latency of a point's reads, with a
+// wavefront a SIMD: 18720 points take 35 us and the sum over chunks 6; one launch a
+// matrix, a thread an element and every operand from L2 took 58 + 16 each, seven times.
+constexpr int kGradTile = 32;
+
+template <int K, int H>
+__global__ void __launch_bounds__(256) grad_partial(const float *__restrict__ X, const float *__restrict__ H1,
+                                                    const float *__restrict__ H2, const float *__restrict__ D1,
+                                                    const float *__restrict__ D2, const float *__restrict__ D3, long N,
+                                                    long chunk, double *__restrict__ partial)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= a * b) return;
-    const int i = e / b, j = e - i * b;
-    const long n0 = blockIdx.y * chunk, n1 = min(N, n0 + chunk);
-    double s = 0.0;
-    for (long n = n0; n < n1; n++) s += (double)A[n * a + i] * (B ? (double)B[n * b + j] : 1.0);
-    partial[(size_t)blockIdx.y * a * b + e] = s;
+    static_assert(H == 64 && K == 32, "256 threads cover a 64 x 64 and a 64 x 32 matrix");
+    __shared__ __attribute__((aligned(16))) float sx[kGradTile * K], sh1[kGradTile * H], sh2[kGradTile * H],
+        sd1[kGradTile * H], sd2[kGradTile * H], sd3[kGradTile];
+    const int t = threadIdx.x, row = t / 16 * 4, c2 = t % 16 * 4, c1 = t % 16 * 2, lane = t & 63, wave = t >> 6;
+    double g2[4][4] = {}, g1[4][2] = {}, col = 0.0;
+    const long n0 = blockIdx.x * chunk, n1 = min(N, n0 + chunk);
+    for (long base = n0; base < n1; base += kGradTile) {
+        const int rows = (int)min((long)kGradTile, n1 - base);
+        for (int q = t; q < rows * H; q += 256) {
+            sh1[q] = H1[base * H + q];
+            sh2[q] = H2[base * H + q];
+            sd1[q] = D1[base * H + q];
+            sd2[q] = D2[base * H + q];
+        }
+        for (int q = t; q < rows * K; q += 256) sx[q] = X[base * K + q];
+        if (t < rows) sd3[t] = D3[base + t];
+        __syncthreads();
+        for (int n = 0; n < rows; n++) {
+            const float4 a2 = *(const float4 *)(sd2 + n * H + row), b2 = *(const float4 *)(sh1 + n * H + c2);
+            const float4 a1 = *(const float4 *)(sd1 + n * H + row);
+            const float2 b1 = *(const float2 *)(sx + n * K + c1);
+            const double p2[4] = {a2.x, a2.y, a2.z, a2.w}, q2[4] = {b2.x, b2.y, b2.z, b2.w};
+            const double p1[4] = {a1.x, a1.y, a1.z, a1.w}, q1[2] = {b1.x, b1.y};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) g2[i][j] = fma(p2[i], q2[j], g2[i][j]);
+#pragma unroll
+                for (int j = 0; j < 2; j++) g1[i][j] = fma(p1[i], q1[j], g1[i][j]);
+            }
+            // column sums: b1, b2 and w3 by a wavefront each, b3 and the squares by two lanes of the last
+            const double d3 = sd3[n];
+            if (wave == 0) col += sd1[n * H + lane];
+            else if (wave == 1) col += sd2[n * H + lane];
+            else if (wave == 2) col = fma((double)sh2[n * H + lane], d3, col);
+            else col = fma(d3, lane ? d3 : 1.0, col);
+        }
+        __syncthreads();
+    }
+    double *const out = partial + (size_t)blockIdx.x * (param_count<K, H>() + 1);
+    double *const oW2 = out + H * K + H, *const ob2 = oW2 + H * H;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) oW2[(row + i) * H + c2 + j] = g2[i][j];
+#pragma unroll
+        for (int j = 0; j < 2; j++) out[(row + i) * K + c1 + j] = g1[i][j];
+    }
+    if (wave == 0) out[H * K + lane] = col;
+    else if (wave == 1) ob2[lane] = col;
+    else if (wave == 2) ob2[H + lane] = col;
+    else if (lane < 2) ob2[2 * H + lane] = col;
 }
 
-__global__ void sum_chunks(const double *__restrict__ partial, int nchunk, int m, double *__restrict__ out)
+// out[e] = sum of the chunks' partials: 16 threads an element, each over every 16th
+// chunk, then in order
+__global__ void __launch_bounds__(1024) sum_chunks(const double *__restrict__ partial, int nchunk, int m,
+                                                   double *__restrict__ out)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= m) return;
+    __shared__ double sm[16][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
     double s = 0.0;
-    for (int c = 0; c < nchunk; c++) s += partial[(size_t)c * m + e];
+    if (e < m)
+#pragma unroll 8
+        for (int c = part; c < nchunk; c += 16) s += partial[(size_t)c * m + e];
+    sm[part][lane] = s;
+    __syncthreads();
+    if (part || e >= m) return;
+    for (int k = 1; k < 16; k++) s += sm[k][lane];
     out[e] = s;
 }
 
@@ -219,9 +327,10 @@ hipError_t launch_mlp_features(const double4 *img, int nimg, const int G[3], con
                                double rf, float *out, int *overflow, hipStream_t st)
 {
     if (K != kMlpK || kRad + kAng != kMlpK) return hipErrorInvalidValue;
-    const long n = (long)G[0] * G[1] * G[2];
-    hipLaunchKernelGGL(mlp_features, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, img, nimg, G[0], G[1],
-                       G[2], h[0], h[1], h[2], R[0], R[1], R[2], rf, out, overflow);
+    unsigned blocks = 1;
+    for (int d = 0; d < 3; d++) blocks *= (G[d] + kBrick[d] - 1) / kBrick[d];
+    hipLaunchKernelGGL(mlp_features, dim3(blocks), dim3(256), 0, st, img, nimg, G[0], G[1], G[2], h[0], h[1], h[2], R[0],
+                       R[1], R[2], rf, out, overflow);
     return hipGetLastError();
 }
 
@@ -244,14 +353,17 @@ hipError_t launch_mlp_deltas(const float *Z1, const float *Z2, const float *Y, c
     return hipGetLastError();
 }
 
-hipError_t launch_outer_sum(const float *A, int a, const float *B, int b, long N, double *partial, int nchunk, double *out,
-                            hipStream_t st)
+// Chunks of the gradient sums: one a CU where each then has 32 points or more
+int mlp_grad_chunks(long N) { return (int)std::max<long>(1, std::min<long>(256, N / kGradTile)); }
+
+hipError_t launch_mlp_grad(const float *X, const float *H1, const float *H2, const float *D1, const float *D2,
+                           const float *D3, long N, double *partial, double *out, hipStream_t st)
 {
-    const long chunk = (N + nchunk - 1) / nchunk;
-    const int m = a * b;
-    hipLaunchKernelGGL(outer_partial, dim3((unsigned)((m + 255) / 256), (unsigned)nchunk), dim3(256), 0, st, A, a, B, b, N,
-                       chunk, partial);
-    hipLaunchKernelGGL(sum_chunks, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, partial, nchunk, m, out);
+    if (N <= 0) return hipErrorInvalidValue;
+    const int nchunk = mlp_grad_chunks(N), m = mlp_param_count(kMlpK, kMlpH) + 1;
+    hipLaunchKernelGGL((grad_partial<kMlpK, kMlpH>), dim3(nchunk), dim3(256), 0, st, X, H1, H2, D1, D2, D3, N,
+                       (N + nchunk - 1) / nchunk, partial);
+    hipLaunchKernelGGL(sum_chunks, dim3((m + 63) / 64), dim3(1024), 0, st, partial, nchunk, m, out);
     return hipGetLastError();
 }
 
