@@ -812,16 +812,18 @@ static int setup_resident(sq_ctx *c)
     for (ResImage &r : v) {
         r.off = (int)pairs;
         pairs += (int64_t)r.dim[0] * r.dim[1] * (r.dim[2] + 2 * kResPad);
-        if (pairs >= (int64_t)1 << 30) return SQ_OK;   // pairs are indexed by int
+        if (pairs >= (int64_t)1 << 28) return SQ_OK;   // the kernel's byte offsets hold 32 bits
     }
     // as many planes of v in LDS as fit, in whole chunks of planes: half the LDS for the
     // small workgroup, two of which share a CU
-    const size_t limit = wg == 512 ? c->lds_limit / 2 : c->lds_limit;
-    int nl = S.nloc[2];
+    int nl = 0;
     size_t total = 0, dynamic = 0;
-    for (; nl > 0; nl--) {
-        resident_lds(S.nloc, nl, &total, &dynamic);
-        if (total <= limit && (nl == S.nloc[2] || nl % 4 == 0)) break;
+    for (size_t limit : {wg == 512 ? c->lds_limit / 2 : c->lds_limit, (size_t)c->lds_limit}) {
+        for (nl = S.nloc[2]; nl > 0; nl--) {
+            resident_lds(S.nloc, nl, &total, &dynamic);
+            if (total <= limit && (nl == S.nloc[2] || nl % 4 == 0)) break;
+        }
+        if (nl > 0) break;
     }
     if (nl < 1 || v.empty()) return SQ_OK;
     int rc;

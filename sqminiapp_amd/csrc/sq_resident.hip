@@ -6,11 +6,11 @@
 //          column in registers, indexed statically (the z loops are unrolled to
 //          NZ planes and guarded by the cube's nz).
 // Per step: gather (one wavefront an image, image by image from a ticket) ->
-// alpha -> r := -b r, scatter of chi alpha into r -> march over the planes,
-// r += (L + diag) v: a plane staged in LDS inside a zero halo gives the x and y
-// neighbours, and its own value is pushed into the thirteen planes of r that it
-// neighbours in z, so no window of v is held -> a = <v, r>, r -= a v, ||r||, v
-// and r change places.  a is taken from r = H v - b v_prev, Paige's form of the
+// alpha -> r := -b r, scatter of chi alpha into r -> march over the planes, two at
+// a time, r += (L + diag) v: the pair staged in LDS inside a zero halo gives the x
+// and y neighbours, and its own values are pushed into the planes of r that they
+// neighbour in z, so no window of v is held -> a = <v, r>, r -= a v, ||r||, v and r
+// change places.  a is taken from r = H v - b v_prev, Paige's form of the
 // recurrence: it equals <v, H v> up to rounding, v being orthogonal to v_prev.
 //
 // What it replaces: the batched kernel streams its vectors (B x 195 KB in FP64)
@@ -91,9 +91,16 @@ __device__ __forceinline__ double group_sum(double x, double *red)
     return lane_value(s, 0);
 }
 
-// LDS row pitch of the staged plane: a halo of 6 on both sides fits to 33 columns,
-// and on a 29-column cube lanes that cross a row's end stay on consecutive banks
+// LDS row pitch of the staged pair of planes: a halo of 6 on both sides fits to 33
+// columns, and on a 29-column cube lanes that cross a row's end stay on consecutive banks.
+// A pair brings both planes' neighbour in one read, which costs no more than the read
+// of one plane's (29^3: march 63 thousand clocks a step plane by plane).
 constexpr int kPitch = 45;
+
+// Staged pairs of planes at a time: with two a plane pair costs one barrier, which is
+// worth the planes of v it takes from LDS (29^3: march 57 -> 48 thousand clocks a step, the
+// other phases 7 more) where one workgroup has the CU to itself.
+constexpr int stage_buffers(int wg) { return wg == 1024 ? 2 : 1; }
 
 // The launch parameters read afresh from the kernel-argument segment: each phase
 // of a step takes its own opaque view, so its scalars live in that phase only.
@@ -134,7 +141,7 @@ template <int WG, int NZ>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) lanczos_resident(ResParams)
 {
     constexpr int NW = WG / 64, O = 6, NLM = 6, MW = kResMaxImages / 32;
-    constexpr int PX = kPitch;
+    constexpr int PX = kPitch, NB = stage_buffers(WG);
     // planes a gather trip loads ahead: what the registers hold beside the column r
     constexpr int UG = 4;
     constexpr int UC = 4;   // planes of a scatter group
@@ -145,6 +152,8 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
     typedef __attribute__((address_space(3))) double ST;
     typedef __attribute__((address_space(1))) double GT;
     typedef const __attribute__((address_space(1))) V2 GV2;
+    typedef const __attribute__((address_space(1))) char GC;   // the table by 32-bit byte offsets
+    typedef __attribute__((address_space(3))) V2 SV2;
     __shared__ ResLds S;
     extern __shared__ __align__(16) unsigned char smem[];
     ST *const vl = (ST *)smem;   // [nl][ncol], then the two staged planes
@@ -175,8 +184,8 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
         live = wave * 64 < ncol;
         const int col = has ? tid : ncol - 1;
         cij = col / nx << 16 | (col % nx);
-        ST *const stage = vl + P->nl * ncol;
-        for (int q = tid; q < 2 * PX * (ny + 2 * O); q += WG) stage[q] = 0;   // the halo stays zero
+        ST *const stage = vl + ((P->nl * ncol + 1) & ~1);
+        for (int q = tid; q < 2 * NB * PX * (ny + 2 * O); q += WG) stage[q] = 0;   // the halo stays zero
     }
     int q_at = 0;
     for (;;) {
@@ -331,7 +340,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 const ParamView P = params();
                 const int nx = P->nloc[0], ny = P->nloc[1], nz = P->nloc[2], nl = P->nl, ncol = nx * ny;
                 const GT *const gvn = (const GT *)P->scratch + ((long)blockIdx.x * (nz - nl) - nl) * ncol;
-                GV2 *const tab = (GV2 *)P->tab;
+                const GC *const tab = (const GC *)P->tab;
                 const double hx = P->hgrid[0], hy = P->hgrid[1], hz = P->hgrid[2];
                 const float rt2 = P->rt2;
                 for (;;) {
@@ -341,13 +350,14 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                     if (li >= nimg) break;
                     const int lo = __builtin_amdgcn_readfirstlane(S.lo[li]), dm = __builtin_amdgcn_readfirstlane(S.dim[li]);
                     const int lx = (signed char)(lo & 255), ly = (signed char)(lo >> 8 & 255), lz = (signed char)(lo >> 16 & 255);
-                    const int dx = dm & 255, dy = dm >> 8 & 255, dz = dm >> 16 & 255, tstep = dx * dy;
+                    const int dx = dm & 255, dy = dm >> 8 & 255, dz = dm >> 16 & 255;
+                    const unsigned ts = dx * dy * 16u;
                     const int x0 = max(lx, 0), nbx = min(lx + dx, nx) - x0;
                     const int y0 = max(ly, 0), nby = min(ly + dy, ny) - y0;
                     const int z0 = max(lz, 0), z1 = min(lz + dz, nz);
                     const int nxy = nbx * nby;
                     const float inv = 1.0f / (float)nbx;
-                    const int off = __builtin_amdgcn_readfirstlane(S.off[li]) + z0 * tstep;
+                    const int off = __builtin_amdgcn_readfirstlane(S.off[li]) + z0 * dx * dy;
                     const double oz = lane_value(S.org[li][2], 0);
                     double acc[NLM];
 #pragma unroll
@@ -358,10 +368,11 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                         const int cx = x0 + q - yi * nbx, cy = y0 + yi;
                         const double x = S.org[li][0] + hx * cx, y = S.org[li][1] + hy * cy;
                         if (q0 + lane >= nxy || !((float)x * (float)x + (float)y * (float)y < rt2)) continue;
-                        int tp = off + cy * dx + cx, vp = z0 * ncol + cy * nx + cx;
+                        unsigned tp = (off + cy * dx + cx) * 16u;
+                        int vp = z0 * ncol + cy * nx + cx;
                         double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-                        auto add = [&](V2 t, double v, int z) {
-                            const double zz = (oz + hz * z);
+                        auto add = [&](V2 t, double v, double z) {
+                            const double zz = fma(hz, z, oz);
                             const double p = t.y * v, pz = p * zz;
                             s0 = fma(t.x, v, s0);
                             s1 += p;
@@ -369,6 +380,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                             s3 = fma(pz, zz, s3);
                         };
                         auto walk = [&](int z, int zb, auto v) {
+                            double zd = z;
 #pragma unroll 1
                             for (; z < zb; z += UG) {
                                 V2 t[UG];
@@ -376,15 +388,16 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
 #pragma unroll
                                 for (int u = 0; u < UG; u++)
                                     if (z + u < zb) {   // uniform
-                                        t[u] = tab[tp + u * tstep];
+                                        t[u] = *(GV2 *)(tab + (tp + u * ts));
                                         vv[u] = v[vp + u * ncol];
                                     }
 #pragma unroll
                                 for (int u = 0; u < UG; u++)
-                                    if (z + u < zb) add(t[u], vv[u], z + u);
+                                    if (z + u < zb) add(t[u], vv[u], zd + u);
                                 const int n = min(UG, zb - z);
-                                tp += n * tstep;
+                                tp += n * ts;
                                 vp += n * ncol;
+                                zd += UG;
                             }
                         };
                         if (z0 < nl) walk(z0, min(z1, nl), vl);
@@ -450,7 +463,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
             if (live) {
                 const ParamView P = params();
                 const int nz = P->nloc[2];
-                GV2 *const tab = (GV2 *)P->tab;
+                const GC *const tab = (const GC *)P->tab;
                 const double hz = P->hgrid[2];
                 int cc = cij;
                 SQ_OPAQUE_V(cc);
@@ -469,7 +482,8 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                         const int li = (wd << 5) + __ffs(m) - 1;
                         m &= m - 1u;
                         const int lo = S.lo[li], dm = S.dim[li];
-                        const int dx = dm & 255, tstep = (dm >> 8 & 255) * dx;
+                        const int dx = dm & 255;
+                        const unsigned ts = (dm >> 8 & 255) * dx * 16u;
                         const double *k6 = reinterpret_cast<const double *>(S.A[li]);
                         const double oz = S.org[li][2];
                         const double x = (S.org[li][0] + xi), y = (S.org[li][1] + yj);
@@ -483,22 +497,22 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                         const int lz = (signed char)(lo >> 16 & 255);
                         const int zl = max(max(lz, 0), (int)ceilf(((float)-oz - half) * ihz));
                         const int zh = min(min(lz + (dm >> 16 & 255), nz) - 1, (int)floorf(((float)-oz + half) * ihz));
-                        int tp = S.off[li] + cj * dx + ci;
+                        unsigned tp = (S.off[li] + cj * dx + ci) * 16u;
 #pragma unroll
                         for (int z0 = 0; z0 < NZ; z0 += UC) {
                             if (zl < z0 + UC && zh >= z0) {
                                 V2 t[UC];
 #pragma unroll
-                                for (int u = 0; u < UC; u++) t[u] = tab[tp + u * tstep];
-                                const double zr = (oz + hz * z0);
+                                for (int u = 0; u < UC; u++) t[u] = *(GV2 *)(tab + (tp + u * ts));
+                                const double zr = fma(hz, (double)z0, oz);
 #pragma unroll
                                 for (int u = 0; u < UC; u++)
                                     if (z0 + u < NZ) {
-                                        const double z = zr + u * hz;
+                                        const double z = fma(hz, (double)u, zr);
                                         r[z0 + u] = fma(t[u].x, k0, fma(t[u].y, fma(z, fma(z, p2, p1), p0), r[z0 + u]));
                                     }
                             }
-                            tp += UC * tstep;
+                            tp += UC * ts;
                         }
                     }
                 }
@@ -511,12 +525,13 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                 const GT *const diag = (const GT *)P->diag_ext;
                 const int eplane = P->extn[1] * P->extn[0];
                 const int sbuf = PX * (P->nloc[1] + 2 * O);
+                SV2 *const stage = (SV2 *)(vl + ((nl * ncol + 1) & ~1));
                 int cc = cij;
                 SQ_OPAQUE_V(cc);
                 const int ci = cc & 0xffff, cj = cc >> 16, col = cj * P->nloc[0] + ci;
                 // the stencil footprint's top-left corner in the staged plane: every neighbour
                 // lies at a constant non-negative offset
-                ST *const scol = vl + nl * ncol + cj * PX + ci;
+                SV2 *const scol = stage + cj * PX + ci;
                 double wt[3][O];
 #pragma unroll
                 for (int d = 0; d < 3; d++)
@@ -524,44 +539,56 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
                     for (int l = 0; l < O; l++) wt[d][l] = P->cw[d][l + 1];
                 const double s = sv;
                 if (live) {
-                    // plane pointers advance as scalars; vl's plane offset likewise
-                    const GT *dp = diag + ebase, *gp = gvn;
+                    // Two planes at a time, staged side by side: a 16-byte read brings a neighbour
+                    // of both.  Plane pointers advance as scalars; vl's plane offset likewise.  The
+                    // pair's second plane may lie past the cube: it is zero then.
                     const int dcol = cj * P->extn[0] + ci;
-                    int zo = 0;
-                    double nxt, dgn = dp[(unsigned)dcol];
-                    if (0 < nl) nxt = vl[col];
-                    else nxt = gp[(unsigned)col];
+                    // v and the diagonal at plane z, or at the last; z is opaque, so no plane's
+                    // addresses are worked out before its turn
+                    auto load = [&](int z, double &v, double &d) {
+                        SQ_OPAQUE(z);
+                        const int k = min(z, nz - 1);
+                        d = (diag + (ebase + k * eplane))[(unsigned)dcol];
+                        if (k < nl) v = vl[k * ncol + col];
+                        else v = (gvn + k * ncol)[(unsigned)col];
+                    };
+                    double n0, n1, d0, d1;
+                    load(0, n0, d0);
+                    load(1, n1, d1);
 #pragma unroll
-                    for (int z = 0; z < NZ; z++) {
+                    for (int z = 0; z < NZ; z += 2) {
                         if (z < nz) {   // uniform
-                            ST *const pl = z & 1 ? scol + sbuf : scol;
-                            const double dg = dgn, vc = s * nxt;
-                            pl[O * PX + O] = vc;
-                            zo += ncol;
-                            gp += ncol;
-                            dp += eplane;
-                            SQ_OPAQUE(zo);
-                            SQ_OPAQUE(gp);
-                            SQ_OPAQUE(dp);
-                            if (z + 1 < nz) {
-                                if (z + 1 < nl) nxt = vl[zo + col];
-                                else nxt = gp[(unsigned)col];
-                                dgn = dp[(unsigned)dcol];
-                            }
+                            const double va = s * n0, vb = z + 1 < nz ? s * n1 : 0.0, da = d0, db = d1;
+                            SV2 *const sc = NB == 2 && (z & 2) ? scol + sbuf : scol;
+                            if (NB == 1 && z) __syncthreads();   // the last pair has been read
+                            sc[O * PX + O] = V2{va, vb};
+                            load(z + 2, n0, d0);
+                            load(z + 3, n1, d1);
                             __syncthreads();
-                            double sx = dg * vc, sy = 0;
+                            double xa = da * va, xb = db * vb, ya = 0, yb = 0;
 #pragma unroll
                             for (int l = 1; l <= O; l++) {
-                                sx = fma(wt[0][l - 1], pl[O * PX + O - l] + pl[O * PX + O + l], sx);
-                                sy = fma(wt[1][l - 1], pl[(O - l) * PX + O] + pl[(O + l) * PX + O], sy);
-                                if (z - l >= 0) r[z >= l ? z - l : 0] = fma(wt[2][l - 1], vc, r[z >= l ? z - l : 0]);
-                                if (z + l < NZ) r[z + l < NZ ? z + l : 0] = fma(wt[2][l - 1], vc, r[z + l < NZ ? z + l : 0]);
+                                const V2 xm = sc[O * PX + O - l], xp = sc[O * PX + O + l];
+                                const V2 ym = sc[(O - l) * PX + O], yp = sc[(O + l) * PX + O];
+                                xa = fma(wt[0][l - 1], xm.x + xp.x, xa);
+                                xb = fma(wt[0][l - 1], xm.y + xp.y, xb);
+                                ya = fma(wt[1][l - 1], ym.x + yp.x, ya);
+                                yb = fma(wt[1][l - 1], ym.y + yp.y, yb);
+                                if (z - l >= 0) r[z >= l ? z - l : 0] = fma(wt[2][l - 1], va, r[z >= l ? z - l : 0]);
+                                if (z + l < NZ) r[z + l < NZ ? z + l : 0] = fma(wt[2][l - 1], va, r[z + l < NZ ? z + l : 0]);
+                                if (z + 1 - l >= 0 && z + 1 < NZ)
+                                    r[z + 1 >= l ? z + 1 - l : 0] = fma(wt[2][l - 1], vb, r[z + 1 >= l ? z + 1 - l : 0]);
+                                if (z + 1 + l < NZ) r[z + 1 + l < NZ ? z + 1 + l : 0] = fma(wt[2][l - 1], vb, r[z + 1 + l < NZ ? z + 1 + l : 0]);
                             }
-                            r[z] += sx + sy;
+                            r[z] += xa + ya;
+                            if (z + 1 < NZ) r[z + 1 < NZ ? z + 1 : 0] += xb + yb;
                         }
                     }
                 } else {
-                    for (int z = 0; z < nz; z++) __syncthreads();   // the staged planes of the others
+                    for (int z = 0; z < nz; z += 2) {   // the staged planes of the others
+                        if (NB == 1 && z) __syncthreads();
+                        __syncthreads();
+                    }
                 }
             }
             // ---- a = <v, r>; r -= a v; ||r||; the vectors change places
@@ -682,7 +709,8 @@ int resident_workgroup(const int nloc[3])
 
 void resident_lds(const int nloc[3], int nl, size_t *total, size_t *dynamic)
 {
-    *dynamic = ((size_t)nl * nloc[0] * nloc[1] + 2 * (size_t)kPitch * (nloc[1] + 12)) * sizeof(double);
+    const size_t vdoubles = (size_t)nl * nloc[0] * nloc[1], pair = 2 * (size_t)kPitch * (nloc[1] + 12);
+    *dynamic = ((vdoubles + 1) / 2 * 2 + stage_buffers(resident_workgroup(nloc)) * pair) * sizeof(double);
     *total = *dynamic + sizeof(ResLds);
 }
 
