@@ -2407,19 +2407,15 @@ std::vector<double4> mlp_images(const System &S, double rf)
     return out;
 }
 
-// descriptors of the context's cell into a device buffer (ng * K floats)
-int mlp_descriptors_dev(sq_ctx *c, double rf, float *dout)
+// descriptors of the context's cell into a device buffer (ng * K floats); dimg: room for the images
+// on the device, dover: for a counter
+int mlp_descriptors_dev(sq_ctx *c, double rf, const std::vector<double4> &img, double4 *dimg, int *dover, float *dout)
 {
     const System &S = c->sys;
-    int G[3], rc;
+    int G[3], rc, over = 0;
     if ((rc = cell_dims(c, G))) return rc;
-    std::vector<double4> img = mlp_images(S, rf);
-    DevBufs B;
-    double4 *dimg;
-    int *dover, over = 0;
-    if ((rc = B.get(&dimg, img.size())) || (rc = B.get(&dover, 1))) return rc;
-    HIP_TRY(hipMemcpy(dimg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(dover, 0, sizeof(int)));
+    HIP_TRY(hipMemcpyAsync(dimg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(launch_zero_int(dover, 1, c->stream));
     const double h[3] = {S.h[0], S.h[1], S.h[2]}, R[3] = {S.range[0], S.range[1], S.range[2]};
     HIP_TRY(launch_mlp_features(dimg, (int)img.size(), G, h, R, kMlpK, rf, dout, dover, c->stream));
     HIP_TRY(hipMemcpyAsync(&over, dover, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -2519,9 +2515,14 @@ int sq_mlp_descriptors(sq_ctx *c, float *out)
     if ((rc = cell_dims(c, G))) return rc;
     HIP_TRY(hipSetDevice(c->device));
     const long ng = (long)G[0] * G[1] * G[2];
+    const std::vector<double4> img = mlp_images(c->sys, kMlpRf);
     DevBufs B;
     float *d;
-    if ((rc = B.get(&d, ng * kMlpK)) || (rc = mlp_descriptors_dev(c, kMlpRf, d))) return rc;
+    double4 *dimg;
+    int *dover;
+    if ((rc = B.get(&d, ng * kMlpK)) || (rc = B.get(&dimg, img.size())) || (rc = B.get(&dover, 1)) ||
+        (rc = mlp_descriptors_dev(c, kMlpRf, img, dimg, dover, d)))
+        return rc;
     HIP_TRY(hipMemcpy(out, d, ng * kMlpK * sizeof(float), hipMemcpyDeviceToHost));
     return SQ_OK;
 }
@@ -2681,10 +2682,15 @@ int sq_mlp_guess(sq_mlp *m, sq_ctx *c, int bf16, double *rho0)
     if (m->device == c->device) {   // the descriptors stay on the device
         HIP_TRY(hipSetDevice(m->device));
         MlpSpace space(m);
+        const std::vector<double4> img = mlp_images(S, kMlpRf);
         const size_t rows = ng;
-        if ((rc = space.reserve(space.piece(rows * kMlpK * 4) + space.piece(rows * 4) + 2 * space.piece(kMlpK * 4)))) return rc;
+        if ((rc = space.reserve(space.piece(rows * kMlpK * 4) + space.piece(rows * 4) + 2 * space.piece(kMlpK * 4) +
+                                space.piece(img.size() * sizeof(double4)) + space.piece(4))))
+            return rc;
         float *const d = space.get<float>(rows * kMlpK);
-        if ((rc = mlp_descriptors_dev(c, kMlpRf, d)) || (rc = mlp_forward_rows(m, space, nullptr, d, ng, bf16, 1, y.data())))
+        double4 *const dimg = space.get<double4>(img.size());
+        int *const dover = space.get<int>(1);
+        if ((rc = mlp_descriptors_dev(c, kMlpRf, img, dimg, dover, d)) || (rc = mlp_forward_rows(m, space, nullptr, d, ng, bf16, 1, y.data())))
             return rc;
     } else {
         std::vector<float> f(ng * kMlpK);

@@ -11,16 +11,17 @@
 //            over eta in {0.005, 0.02}, zeta in {1, 2, 4, 16}, lam = +-1 (16 functions)
 //   y = w3 . silu(W2 silu(W1 xhat + b1) + b2) + b3,  xhat = (f - mean) * rstd,  silu(z) = z/(1 + e^-z)
 // Parameters packed W1[H][K], b1[H], W2[H][H], b2[H], w3[H], b3 (6337 floats
-// for K = 32, H = 64): they sit in LDS; one thread carries one point through
-// the layers with FMA chains.  The layers are 32x64 and 64x64 -- far below an
-// MFMA tile's worth of reuse per point -- and the whole forward over a cell is
-// microseconds, so plain FMA is the right tool here.
+// for K = 32, H = 64): they sit in LDS, and FMA chains carry a point through the
+// layers.  The layers are 32x64 and 64x64 -- far below an MFMA tile's worth of reuse
+// per point -- and the whole forward over a cell is microseconds, so plain FMA is the
+// right tool here.
 // Training (FP32, full batch): deltas per point, then all gradient sums over points
 // in one pass over point chunks, with double partial sums and a fixed-order second
 // pass (deterministic), then Adam.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "sq_kernels.h"
 
@@ -144,78 +145,141 @@ __device__ __forceinline__ float dsilu(float z)
     return sg * (1.0f + z * (1.0f - sg));
 }
 
+// A point's layers by four wavefronts, a quarter of each layer's outputs a wavefront
+// (a lane a point, 64 points a block), four outputs' chains side by side; the
+// activations change hands through LDS.  Each output's chain runs over its inputs in
+// order.  Bound by the chains' latency where the rows are few: 18720 rows take 30 us, and
+// 60 with a point's whole network in one thread; 153504 rows in BF16 86 and 89.
+constexpr int kPts = 64, kOut = 4;   // points of a block; outputs side by side
+
 template <int K, int H, bool B16>
 __global__ void __launch_bounds__(256) mlp_forward(const float *__restrict__ X, long N, const float *__restrict__ P,
                                                    const float *__restrict__ mean, const float *__restrict__ rstd,
                                                    float *__restrict__ H1, float *__restrict__ H2, float *__restrict__ Z1,
                                                    float *__restrict__ Z2, float *__restrict__ Y)
 {
-    constexpr int NP = param_count<K, H>();
-    __shared__ float w[NP];
+    constexpr int NP = param_count<K, H>(), Q = H / 4;
+    static_assert(K % 4 == 0 && Q % kOut == 0, "rows of four weights, quarters of four outputs");
+    __shared__ __attribute__((aligned(16))) float w[NP];
+    __shared__ float ex[H][kPts];
     for (int q = threadIdx.x; q < NP; q += blockDim.x) w[q] = B16 ? to_bf16(P[q]) : P[q];
-    __syncthreads();
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
+    const int lane = threadIdx.x & 63, o0 = (threadIdx.x >> 6) * Q;
+    const long n = (long)blockIdx.x * kPts + lane;
+    const bool has = n < N;
     const float *W1 = w, *b1 = W1 + H * K, *W2 = b1 + H, *b2 = W2 + H * H, *w3 = b2 + H, *b3 = w3 + H;
-    float xh[K];
+    float a[H];   // inputs of the layer at hand
+    {
+        const float *x = X + (has ? n : N - 1) * K;
 #pragma unroll
-    for (int q = 0; q < K; q++) {
-        float v = X[n * K + q];
-        if (mean) v = (v - mean[q]) * rstd[q];
-        xh[q] = B16 ? to_bf16(v) : v;
+        for (int q = 0; q < K; q++) {
+            float v = x[q];
+            if (mean) v = (v - mean[q]) * rstd[q];
+            a[q] = B16 ? to_bf16(v) : v;
+        }
     }
-    float a1[H];
+    __syncthreads();
+    // outputs o .. o + kOut - 1 of a layer with M inputs
+    auto chains = [&](const float *W, const float *b, auto M, int o, float s[kOut]) {
+        constexpr int n_in = decltype(M)::value;
 #pragma unroll
-    for (int i = 0; i < H; i++) {
-        float s = b1[i];
+        for (int k = 0; k < kOut; k++) s[k] = b[o + k];
 #pragma unroll
-        for (int q = 0; q < K; q++) s = fmaf(W1[i * K + q], xh[q], s);
-        const float t = silu(s);
-        a1[i] = B16 ? to_bf16(t) : t;
-        if (H1) H1[n * H + i] = a1[i];
-        if (Z1) Z1[n * H + i] = s;
+        for (int q = 0; q < n_in; q += 4)
+#pragma unroll
+            for (int k = 0; k < kOut; k++) {
+                const float4 c = *reinterpret_cast<const float4 *>(W + (o + k) * n_in + q);
+                s[k] = fmaf(c.x, a[q], s[k]);
+                s[k] = fmaf(c.y, a[q + 1], s[k]);
+                s[k] = fmaf(c.z, a[q + 2], s[k]);
+                s[k] = fmaf(c.w, a[q + 3], s[k]);
+            }
+    };
+    // kOut outputs' activations to LDS, and to the rows a backward pass needs
+    auto activate = [&](int o, const float s[kOut], float *Hn, float *Zn) {
+        float t[kOut];
+#pragma unroll
+        for (int k = 0; k < kOut; k++) {
+            t[k] = silu(s[k]);
+            if (B16) t[k] = to_bf16(t[k]);
+            ex[o + k][lane] = t[k];
+        }
+        if (Hn && has) *reinterpret_cast<float4 *>(Hn + n * H + o) = make_float4(t[0], t[1], t[2], t[3]);
+        if (Zn && has) *reinterpret_cast<float4 *>(Zn + n * H + o) = make_float4(s[0], s[1], s[2], s[3]);
+    };
+#pragma unroll 1
+    for (int o = o0; o < o0 + Q; o += kOut) {
+        float s[kOut];
+        chains(W1, b1, std::integral_constant<int, K>(), o, s);
+        activate(o, s, H1, Z1);
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < H; i++) a[i] = ex[i][lane];
+    __syncthreads();
+#pragma unroll 1
+    for (int o = o0; o < o0 + Q; o += kOut) {
+        float s[kOut];
+        chains(W2, b2, std::integral_constant<int, H>(), o, s);
+        activate(o, s, H2, Z2);
+    }
+    __syncthreads();
+    if (o0 || !has) return;
     float y = b3[0];
-    for (int j = 0; j < H; j++) {
-        float s = b2[j];
 #pragma unroll
-        for (int i = 0; i < H; i++) s = fmaf(W2[j * H + i], a1[i], s);
-        float t = silu(s);
-        if (B16) t = to_bf16(t);
-        if (H2) H2[n * H + j] = t;
-        if (Z2) Z2[n * H + j] = s;
-        y = fmaf(w3[j], t, y);
-    }
+    for (int j = 0; j < H; j++) y = fmaf(w3[j], ex[j][lane], y);
     Y[n] = y;
 }
 
-// L = (1/2N) sum (y - t)^2: d3 = (y - t)/N, d2 = d3 w3 silu'(z2), d1 = (W2^T d2) silu'(z1)
+// L = (1/2N) sum (y - t)^2: d3 = (y - t)/N, d2 = d3 w3 silu'(z2), d1 = (W2^T d2) silu'(z1);
+// split as the forward pass (18720 rows: 17 us, and 36 with a point a thread)
 template <int K, int H>
 __global__ void __launch_bounds__(256) mlp_deltas(const float *__restrict__ Z1, const float *__restrict__ Z2,
                                                   const float *__restrict__ Y, const float *__restrict__ T, long N,
                                                   const float *__restrict__ P, float *__restrict__ D1,
                                                   float *__restrict__ D2, float *__restrict__ D3)
 {
-    __shared__ float w2[H * H], w3[H];
+    constexpr int Q = H / 4;
+    __shared__ __attribute__((aligned(16))) float w2[H * H];
+    __shared__ float w3[H], ex[H][kPts];
     const float *W2g = P + H * K + H, *w3g = W2g + H * H + H;
     for (int q = threadIdx.x; q < H * H; q += blockDim.x) w2[q] = W2g[q];
     for (int q = threadIdx.x; q < H; q += blockDim.x) w3[q] = w3g[q];
     __syncthreads();
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    const float d3 = (Y[n] - T[n]) / (float)N;
-    D3[n] = d3;
-    float d2[H];
+    const int lane = threadIdx.x & 63, o0 = (threadIdx.x >> 6) * Q;
+    const long n = (long)blockIdx.x * kPts + lane;
+    const bool has = n < N;
+    const long row = (has ? n : N - 1) * H;
+    const float d3 = has ? (Y[n] - T[n]) / (float)N : 0.0f;
+    if (has && o0 == 0) D3[n] = d3;
 #pragma unroll
-    for (int j = 0; j < H; j++) {
-        d2[j] = d3 * w3[j] * dsilu(Z2[n * H + j]);
-        D2[n * H + j] = d2[j];
+    for (int o = o0; o < o0 + Q; o += kOut) {
+        const float4 z = *reinterpret_cast<const float4 *>(Z2 + row + o);
+        const float zz[kOut] = {z.x, z.y, z.z, z.w};
+        float d[kOut];
+#pragma unroll
+        for (int k = 0; k < kOut; k++) {
+            d[k] = d3 * w3[o + k] * dsilu(zz[k]);
+            ex[o + k][lane] = d[k];
+        }
+        if (has) *reinterpret_cast<float4 *>(D2 + row + o) = make_float4(d[0], d[1], d[2], d[3]);
     }
-    for (int i = 0; i < H; i++) {
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < H; j++) s = fmaf(w2[j * H + i], d2[j], s);
-        D1[n * H + i] = s * dsilu(Z1[n * H + i]);
+    __syncthreads();
+#pragma unroll 1
+    for (int o = o0; o < o0 + Q; o += kOut) {
+        float s[kOut] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 16
+        for (int j = 0; j < H; j++) {
+            const float4 c = *reinterpret_cast<const float4 *>(w2 + j * H + o);
+            const float d = ex[j][lane];
+            s[0] = fmaf(c.x, d, s[0]);
+            s[1] = fmaf(c.y, d, s[1]);
+            s[2] = fmaf(c.z, d, s[2]);
+            s[3] = fmaf(c.w, d, s[3]);
+        }
+        const float4 z = *reinterpret_cast<const float4 *>(Z1 + row + o);
+        if (has)
+            *reinterpret_cast<float4 *>(D1 + row + o) =
+                make_float4(s[0] * dsilu(z.x), s[1] * dsilu(z.y), s[2] * dsilu(z.z), s[3] * dsilu(z.w));
     }
 }
 
@@ -224,7 +288,7 @@ __global__ void __launch_bounds__(256) mlp_deltas(const float *__restrict__ Z1, 
 // points' rows lies in LDS; a thread keeps a 4 x 4 piece of W2 and a 4 x 2 piece of
 // W1 in registers, so a point costs it four LDS reads and 24 multiply-adds, and a
 // column sum is one thread's.  Bound by the latency of a point's reads, with a
-// wavefront a SIMD: 18720 points take 35 us and the sum over chunks 6; one launch a
+// wavefront a SIMD: 18720 points take 33 us and the sum over chunks 6; one launch a
 // matrix, a thread an element and every operand from L2 took 58 + 16 each, seven times.
 constexpr int kGradTile = 32;
 
@@ -251,6 +315,7 @@ __global__ void __launch_bounds__(256) grad_partial(const float *__restrict__ X,
         for (int q = t; q < rows * K; q += 256) sx[q] = X[base * K + q];
         if (t < rows) sd3[t] = D3[base + t];
         __syncthreads();
+#pragma unroll 4
         for (int n = 0; n < rows; n++) {
             const float4 a2 = *(const float4 *)(sd2 + n * H + row), b2 = *(const float4 *)(sh1 + n * H + c2);
             const float4 a1 = *(const float4 *)(sd1 + n * H + row);
@@ -338,7 +403,7 @@ hipError_t launch_mlp_forward(const float *X, long N, const float *P, const floa
                               float *H2, float *Z1, float *Z2, float *Y, int bf16, hipStream_t st)
 {
     if (N <= 0) return hipSuccess;
-    const dim3 g((unsigned)((N + 255) / 256)), b(256);
+    const dim3 g((unsigned)((N + kPts - 1) / kPts)), b(256);
     if (bf16) hipLaunchKernelGGL((mlp_forward<kMlpK, kMlpH, true>), g, b, 0, st, X, N, P, mean, rstd, H1, H2, Z1, Z2, Y);
     else hipLaunchKernelGGL((mlp_forward<kMlpK, kMlpH, false>), g, b, 0, st, X, N, P, mean, rstd, H1, H2, Z1, Z2, Y);
     return hipGetLastError();
@@ -348,7 +413,7 @@ hipError_t launch_mlp_deltas(const float *Z1, const float *Z2, const float *Y, c
                              float *D1, float *D2, float *D3, hipStream_t st)
 {
     if (N <= 0) return hipSuccess;
-    hipLaunchKernelGGL((mlp_deltas<kMlpK, kMlpH>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, Z1, Z2, Y, T, N, P,
+    hipLaunchKernelGGL((mlp_deltas<kMlpK, kMlpH>), dim3((unsigned)((N + kPts - 1) / kPts)), dim3(256), 0, st, Z1, Z2, Y, T, N, P,
                        D1, D2, D3);
     return hipGetLastError();
 }
