@@ -105,9 +105,9 @@ int sq_get_info(sq_ctx *ctx, sq_info *info);
 
 /* Whether FP64 passes run in the resident kernel (one node a workgroup, its
  * vectors on chip): planes = the planes of the current vector it keeps in LDS,
- * 0 where the kernel of sq_info (workgroup, batch, gather_trip: the
- * autotuner's choice among the column-marching kernels, which FP32 passes
- * always take) runs instead. */
+ * 0 where the kernel that sq_info reports runs instead (workgroup, batch,
+ * gather_trip: the autotuner's choice among the column-marching kernels,
+ * which FP32 passes always take). */
 int sq_resident_planes(sq_ctx *ctx, int *planes);
 
 /* V_eff on the global grid (npts[0]*npts[1]*npts[2], i fastest), wrapped
