@@ -2407,23 +2407,6 @@ std::vector<double4> mlp_images(const System &S, double rf)
     return out;
 }
 
-// descriptors of the context's cell into a device buffer (ng * K floats); dimg: room for the images
-// on the device, dover: for a counter
-int mlp_descriptors_dev(sq_ctx *c, double rf, const std::vector<double4> &img, double4 *dimg, int *dover, float *dout)
-{
-    const System &S = c->sys;
-    int G[3], rc, over = 0;
-    if ((rc = cell_dims(c, G))) return rc;
-    HIP_TRY(hipMemcpyAsync(dimg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(launch_zero_int(dover, 1, c->stream));
-    const double h[3] = {S.h[0], S.h[1], S.h[2]}, R[3] = {S.range[0], S.range[1], S.range[2]};
-    HIP_TRY(launch_mlp_features(dimg, (int)img.size(), G, h, R, kMlpK, rf, dout, dover, c->stream));
-    HIP_TRY(hipMemcpyAsync(&over, dover, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (over) return set_err(SQ_ERR_RANGE, "descriptors: more atoms within the cutoff of a point than the kernel holds");
-    return SQ_OK;
-}
-
 }  // namespace
 
 extern "C" {
@@ -2520,9 +2503,16 @@ int sq_mlp_descriptors(sq_ctx *c, float *out)
     float *d;
     double4 *dimg;
     int *dover;
-    if ((rc = B.get(&d, ng * kMlpK)) || (rc = B.get(&dimg, img.size())) || (rc = B.get(&dover, 1)) ||
-        (rc = mlp_descriptors_dev(c, kMlpRf, img, dimg, dover, d)))
-        return rc;
+    if ((rc = B.get(&d, ng * kMlpK)) || (rc = B.get(&dimg, img.size())) || (rc = B.get(&dover, 1))) return rc;
+    const System &S = c->sys;
+    const double h[3] = {S.h[0], S.h[1], S.h[2]}, R[3] = {S.range[0], S.range[1], S.range[2]};
+    int over = 0;
+    HIP_TRY(hipMemcpyAsync(dimg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(launch_zero_int(dover, 1, c->stream));
+    HIP_TRY(launch_mlp_features(dimg, (int)img.size(), G, h, R, kMlpK, kMlpRf, d, dover, c->stream));
+    HIP_TRY(hipMemcpyAsync(&over, dover, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (over) return set_err(SQ_ERR_RANGE, "descriptors: more atoms within the cutoff of a point than the kernel holds");
     HIP_TRY(hipMemcpy(out, d, ng * kMlpK * sizeof(float), hipMemcpyDeviceToHost));
     return SQ_OK;
 }
@@ -2600,24 +2590,11 @@ int sq_mlp_loss_grad(sq_mlp *m, const float *X, const float *T, long N, double *
     return SQ_OK;
 }
 
-// Y (host) of N rows; the rows come from the host, or are already in the device's dX
-static int mlp_forward_rows(sq_mlp *m, MlpSpace &space, const float *X, const float *dX, long N, int bf16, int normalize,
-                            float *Y)
+// mean and rstd of the normalization to the device, one after the other
+static int mlp_put_norm(sq_mlp *m, float *dnorm)
 {
-    const size_t rows = N;
-    if (!dX) {
-        if (int rc = space.reserve(space.piece(rows * m->K * 4) + space.piece(rows * 4) + 2 * space.piece(m->K * 4))) return rc;
-        float *const x = space.get<float>(rows * m->K);
-        HIP_TRY(hipMemcpy(x, X, rows * m->K * sizeof(float), hipMemcpyHostToDevice));
-        dX = x;
-    }
-    float *const dY = space.get<float>(rows), *const dmean = space.get<float>(m->K), *const drstd = space.get<float>(m->K);
-    HIP_TRY(hipMemcpy(dmean, m->mean.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(drstd, m->rstd.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(launch_mlp_forward(dX, N, m->p, normalize ? dmean : nullptr, normalize ? drstd : nullptr, nullptr, nullptr,
-                               nullptr, nullptr, dY, bf16, m->stream));
-    HIP_TRY(hipMemcpyAsync(Y, dY, N * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipStreamSynchronize(m->stream));
+    HIP_TRY(hipMemcpy(dnorm, m->mean.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dnorm + m->K, m->rstd.data(), m->K * sizeof(float), hipMemcpyHostToDevice));
     return SQ_OK;
 }
 
@@ -2626,7 +2603,17 @@ int sq_mlp_forward(sq_mlp *m, const float *X, long N, int bf16, int normalize, f
     if (!m || !X || !Y || N <= 0) return set_err(SQ_ERR_ARG, "bad argument");
     HIP_TRY(hipSetDevice(m->device));
     MlpSpace space(m);
-    return mlp_forward_rows(m, space, X, nullptr, N, bf16, normalize, Y);
+    const size_t rows = N;
+    int rc;
+    if ((rc = space.reserve(space.piece(rows * m->K * 4) + space.piece(rows * 4) + space.piece(2 * m->K * 4)))) return rc;
+    float *const dX = space.get<float>(rows * m->K), *const dY = space.get<float>(rows), *const norm = space.get<float>(2 * m->K);
+    HIP_TRY(hipMemcpy(dX, X, rows * m->K * sizeof(float), hipMemcpyHostToDevice));
+    if ((rc = mlp_put_norm(m, norm))) return rc;
+    HIP_TRY(launch_mlp_forward(dX, N, m->p, normalize ? norm : nullptr, normalize ? norm + m->K : nullptr, nullptr, nullptr,
+                               nullptr, nullptr, dY, bf16, m->stream));
+    HIP_TRY(hipMemcpyAsync(Y, dY, N * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    HIP_TRY(hipStreamSynchronize(m->stream));
+    return SQ_OK;
 }
 
 int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
@@ -2670,6 +2657,63 @@ int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
     return SQ_OK;
 }
 
+// The guess where model and context share a device: descriptors, network, superposed atoms and
+// the two normalizations there, one copy of the density back
+static int mlp_guess_dev(sq_mlp *m, sq_ctx *c, const int G[3], int bf16, double *rho0)
+{
+    const System &S = c->sys;
+    const size_t ng = (size_t)G[0] * G[1] * G[2];
+    const std::vector<double4> img = mlp_images(S, kMlpRf);
+    const std::vector<DensityImage> dimg = density_images(S, G);
+    std::vector<double> tab;
+    std::vector<DensityType> types;
+    for (const Pseudopotential &P : S.psd) {
+        types.push_back({(int)tab.size(), P.size});
+        tab.insert(tab.end(), P.r.begin(), P.r.end());
+        tab.insert(tab.end(), P.s_uu.y.begin(), P.s_uu.y.end());
+        tab.insert(tab.end(), P.s_uu.yd.begin(), P.s_uu.yd.end());
+    }
+    HIP_TRY(hipSetDevice(m->device));
+    MlpSpace W(m);
+    int rc, flags[2];
+    if ((rc = W.reserve(W.piece(ng * kMlpK * 4) + W.piece(ng * 4) + W.piece(2 * kMlpK * 4) + W.piece(img.size() * sizeof(double4)) +
+                        W.piece(sizeof flags) + W.piece(ng * 8) + W.piece(kRedBlocks * 8) + W.piece(2 * 8) +
+                        W.piece(dimg.size() * sizeof(DensityImage)) + W.piece(types.size() * sizeof(DensityType)) +
+                        W.piece(tab.size() * 8))))
+        return rc;
+    float *const X = W.get<float>(ng * kMlpK), *const Y = W.get<float>(ng), *const norm = W.get<float>(2 * kMlpK);
+    double4 *const ximg = W.get<double4>(img.size());
+    int *const xflags = W.get<int>(2);
+    double *const rho = W.get<double>(ng), *const part = W.get<double>(kRedBlocks), *const sums = W.get<double>(2);
+    DensityImage *const rimg = W.get<DensityImage>(dimg.size());
+    DensityType *const rtypes = W.get<DensityType>(types.size());
+    double *const rtab = W.get<double>(tab.size());
+    hipStream_t st = c->stream;
+    if ((rc = mlp_put_norm(m, norm))) return rc;
+    HIP_TRY(hipMemcpyAsync(ximg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(rimg, dimg.data(), dimg.size() * sizeof(DensityImage), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(rtypes, types.data(), types.size() * sizeof(DensityType), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(rtab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    HIP_TRY(launch_zero_int(xflags, 2, st));
+    const double h[3] = {S.h[0], S.h[1], S.h[2]}, R[3] = {S.range[0], S.range[1], S.range[2]};
+    HIP_TRY(launch_mlp_features(ximg, (int)img.size(), G, h, R, kMlpK, kMlpRf, X, xflags, st));
+    HIP_TRY(launch_mlp_forward(X, (long)ng, m->p, norm, norm + kMlpK, nullptr, nullptr, nullptr, nullptr, Y, bf16, st));
+    HIP_TRY(launch_superposed(rimg, (int)dimg.size(), rtypes, rtab, G, h, R, rho, xflags + 1, st));
+    HIP_TRY(launch_dot(rho, nullptr, (long)ng, 1.0, part, kRedBlocks, sums, st));
+    HIP_TRY(launch_guess_add(rho, Y, sums, (double)S.noetot, S.dV, m->tscale, (long)ng, st));
+    HIP_TRY(launch_dot(rho, nullptr, (long)ng, 1.0, part, kRedBlocks, sums + 1, st));
+    HIP_TRY(launch_guess_scale(rho, sums + 1, (double)S.noetot, S.dV, (long)ng, st));
+    double tot;
+    HIP_TRY(hipMemcpyAsync(flags, xflags, sizeof flags, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&tot, sums + 1, sizeof tot, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    if (flags[0]) return set_err(SQ_ERR_RANGE, "descriptors: more atoms within the cutoff of a point than the kernel holds");
+    if (flags[1]) return set_err(flags[1], "atomic density: spline evaluation failed");
+    if (!(tot * S.dV > 0)) return set_err(SQ_ERR_RANGE, "network density has no charge");
+    HIP_TRY(hipMemcpy(rho0, rho, ng * sizeof(double), hipMemcpyDeviceToHost));
+    return SQ_OK;
+}
+
 int sq_mlp_guess(sq_mlp *m, sq_ctx *c, int bf16, double *rho0)
 {
     if (!m || !c || !rho0) return set_err(SQ_ERR_ARG, "null argument");
@@ -2677,25 +2721,10 @@ int sq_mlp_guess(sq_mlp *m, sq_ctx *c, int bf16, double *rho0)
     const System &S = c->sys;
     int G[3], rc;
     if ((rc = cell_dims(c, G))) return rc;
+    if (m->device == c->device) return mlp_guess_dev(m, c, G, bf16, rho0);
     const long ng = (long)G[0] * G[1] * G[2];
-    std::vector<float> y(ng);
-    if (m->device == c->device) {   // the descriptors stay on the device
-        HIP_TRY(hipSetDevice(m->device));
-        MlpSpace space(m);
-        const std::vector<double4> img = mlp_images(S, kMlpRf);
-        const size_t rows = ng;
-        if ((rc = space.reserve(space.piece(rows * kMlpK * 4) + space.piece(rows * 4) + 2 * space.piece(kMlpK * 4) +
-                                space.piece(img.size() * sizeof(double4)) + space.piece(4))))
-            return rc;
-        float *const d = space.get<float>(rows * kMlpK);
-        double4 *const dimg = space.get<double4>(img.size());
-        int *const dover = space.get<int>(1);
-        if ((rc = mlp_descriptors_dev(c, kMlpRf, img, dimg, dover, d)) || (rc = mlp_forward_rows(m, space, nullptr, d, ng, bf16, 1, y.data())))
-            return rc;
-    } else {
-        std::vector<float> f(ng * kMlpK);
-        if ((rc = sq_mlp_descriptors(c, f.data())) || (rc = sq_mlp_forward(m, f.data(), ng, bf16, 1, y.data()))) return rc;
-    }
+    std::vector<float> f(ng * kMlpK), y(ng);
+    if ((rc = sq_mlp_descriptors(c, f.data())) || (rc = sq_mlp_forward(m, f.data(), ng, bf16, 1, y.data()))) return rc;
     std::vector<double> rat;
     double sc;
     Status st = build_atomic_density(S, rat, sc);

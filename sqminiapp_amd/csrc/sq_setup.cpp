@@ -869,6 +869,24 @@ Status local_forces(const System &S, const double *phi, double scale, std::vecto
     return {};
 }
 
+std::vector<DensityImage> density_images(const System &S, const int G[3])
+{
+    std::vector<DensityImage> out;
+    for (const CellImage &im : cell_images(S, G)) {
+        DensityImage d{};
+        bool meets = true;
+        for (int k = 0; k < 3; k++) {
+            d.lo[k] = im.lo[k];
+            d.hi[k] = im.hi[k];
+            d.X[k] = im.X[k];
+            meets = meets && im.lo[k] <= G[k] - 1 && im.hi[k] >= 0;
+        }
+        d.at = im.at;
+        if (meets) out.push_back(d);
+    }
+    return out;
+}
+
 Status build_atomic_density(const System &S, std::vector<double> &rho, double &scale)
 {
     const int G[3] = {S.npts[0] - 1, S.npts[1] - 1, S.npts[2] - 1};

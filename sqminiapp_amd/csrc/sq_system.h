@@ -121,6 +121,13 @@ Status build_system(const std::string &dir, const std::string &name, const Setup
 // densities scaled to N_e.
 Status build_pseudocharge(const System &S, std::vector<double> &b, double &eself, double &scale);
 Status build_atomic_density(const System &S, std::vector<double> &rho, double &scale);
+// The images whose boxes meet the cell, in the order build_atomic_density adds them
+struct DensityImage {
+    int lo[3], hi[3];   // box, unwrapped global indices
+    int at, pad;        // type
+    double X[3];
+};
+std::vector<DensityImage> density_images(const System &S, const int G[3]);
 // Pseudocharge forces F[3 * nAtoms] for the potential phi on the periodic cell
 // (the derivative of (1/2) int phi (b - rho) - E_self at fixed rho; scale is
 // the neutrality factor build_pseudocharge returned).
