@@ -282,8 +282,9 @@ def main():
     b32 = algorithmic_bytes_per_node(I.nqp, I.nc, 4)
     slab_nodes = [slabs[(args.warmup + i) % len(slabs)][1] for i in range(args.steps)]
     achieved = b64 * sum(slab_nodes) / (lz64.sum() * 1e-3) / 1e9
-    traffic = load_json("lanczos_c128_fp64_pmc.json") if args.config == "C128" else None
-    if traffic and (resident or traffic.get("batch") != I.batch[0]):
+    pmc = "lanczos_resident_c128_fp64_pmc.json" if resident else "lanczos_c128_fp64_pmc.json"
+    traffic = load_json(pmc) if args.config == "C128" else None
+    if traffic and traffic.get("batch") != (1 if resident else I.batch[0]):
         traffic = None   # the profile was taken of another FP64 kernel
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
