@@ -142,8 +142,10 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4)))
 {
     constexpr int NW = WG / 64, O = 6, NLM = 6, MW = kResMaxImages / 32;
     constexpr int PX = kPitch, NB = stage_buffers(WG);
-    // planes a gather trip loads ahead: what the registers hold beside the column r
-    constexpr int UG = 4;
+    // planes a gather trip loads ahead: what the registers hold beside the column r (1024 threads,
+    // 29^3: 168.7, 172.8 and 170.9 thousand clocks a step with 3, 4 and 2; 512 threads, 21^3: 99.6
+    // and 98.8 with 3 and 4)
+    constexpr int UG = WG == 1024 ? 3 : 4;
     constexpr int UC = 4;   // planes of a scatter group
     constexpr int UD = 4;   // planes of a dot or update chunk
     typedef double V2 __attribute__((ext_vector_type(2)));
