@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(1024) lanczos_zbatch(KParams P)
     VB *plane = reinterpret_cast<VB *>(smem + P.lds_plane);
     int4 *trun = reinterpret_cast<int4 *>(smem + P.lds_run);          // [img]: first, last image of its atom; type
     double *pshare = reinterpret_cast<double *>(smem + P.lds_share);  // [img][B]: an atom's share of <v, V_nl v>
-    __shared__ int s_count, s_ticket;
+    __shared__ int s_count;
     __shared__ T s_w[3][8];
     __shared__ long s_next;
     __shared__ double s_g[4][kMatsubara][2];
@@ -271,21 +271,12 @@ __global__ void __launch_bounds__(1024) lanczos_zbatch(KParams P)
             s_nq[tid] = P.nqp;
             s_st[tid] = 0;
         }
-        if (tid == 0) {
-            s_alive = (1 << nb) - 1;
-            s_ticket = 0;
-        }
+        if (tid == 0) s_alive = (1 << nb) - 1;
         __syncthreads();
         int checks = 0;
         for (int step = 0; step <= P.nqp && s_alive; step++) {
             // ---- gather on the matrix cores: A[li][n][ch] = sum_{box & cube} v_n chi_ch
-            for (;;) {
-                // image by image from a ticket: boxes clipped by the cube differ in size (dealt out in
-                // turn, the last wavefront's wait was 31 of a step's 555 thousand clocks; now 22)
-                int li = 0;
-                if (lane == 0) li = atomicAdd(&s_ticket, 1);
-                li = __builtin_amdgcn_readfirstlane(li);
-                if (li >= nimg) break;
+            for (int li = wave; li < nimg; li += NW) {
                 const int4 lo = tlo[li], dm = tdim[li];
                 const int nlm = dm.w & 255;
                 const double4 cen = tcen[li];
@@ -503,7 +494,6 @@ __global__ void __launch_bounds__(1024) lanczos_zbatch(KParams P)
 #pragma unroll
             for (int b = 0; b < B; b++) pn[b] = red[(B + 1) * NW + b];
             __syncthreads();
-            if (tid == 0) s_ticket = 0;   // for the next step's gather
             // ---- local part, marching the union planes: u_b = (L + diag) v_b into Bu and <v_b, u_b>
             // <v_b, u_b> and later ||w_b||^2: in FP32 each product is exact in FP64
             // (24 x 24 bits), so the sums are FP64 sums of exact products
