@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(kT) axpbypgz(double alpha, const double *x, do
 // chunks of dot_partial, in the launch that forms its vector; its partials are
 // summed by every block of the next launch, which costs 4 us there where launches of
 // their own for the sum and the scalars cost 35.  The first operands of a block's chunk
-// are on the way meanwhile.  Bound by those chains: 157248 points take 7, 8 and 8 us
+// are on the way meanwhile.  Bound by those chains: 153504 points take 7, 8 and 8 us
 // (86 a step in seven launches), of which their 12 passes over memory are 3.
 template <int ORDER>
 __global__ void __launch_bounds__(kT) cg_ap(const double *__restrict__ p, double *__restrict__ Ap, int G0, int G1, int G2,
