@@ -71,17 +71,19 @@ typedef struct {
     double gamma[8][4];      /* Gamma_l per type, lsdft_initObjs.cc:822-869 */
     double cutoff[8][3];     /* pseudocharge cutoff, lsdft_initObjs.cc:628-817 */
     long long chi_entries;   /* total projector entries over all images */
-    int kernel;              /* Lanczos kernel in use: 1 column-marching, 0 generic */
+    int kernel;              /* Lanczos kernels in use: 1 column-marching (in FP64 also resident), 0 generic */
     int kmax;                /* most images meeting one (x,y) column of a cube */
-    int workgroup[2];        /* Lanczos workgroup size per precision (SQ_FP64, SQ_FP32), chosen by
-                                the autotuner at creation */
+    int workgroup[2];        /* workgroup size of the Lanczos kernel that runs, per precision (SQ_FP64,
+                                SQ_FP32), chosen by the autotuner at creation */
     float tune_ms[2][2];     /* autotuner probe times per precision for 512 and 1024 threads
                                 (0 where not timed) */
-    int batch[2];            /* nodes per Lanczos workgroup per precision: 1 (one-node kernel) or
-                                2, 4 (batched kernel, nodes stacked in z) */
-    int gather_trip[2];      /* batched kernel's gather trip per precision (0: one-node kernel) */
+    int batch[2];            /* the kernel per precision: 0 (resident kernel: one node a workgroup, its
+                                vectors on chip), 1 (one-node kernel) or the nodes stacked in z of a
+                                workgroup, 2 or 4 (batched kernel) */
+    int gather_trip[2];      /* batched kernel's gather trip per precision (0: the others) */
     float tune_candidates_ms[2][6]; /* autotuner probe times per precision: one-node 512 / 1024
-                                threads, B=2 trips a / b, B=4 trips a / b (0: not timed) */
+                                threads, B=2 trips a / b, B=4 trips a / b (0: not timed); the last
+                                of FP64 is the resident kernel's */
     int union_images[2];     /* most images meeting one union cube, B = 2 and B = 4 */
 } sq_info;
 
@@ -103,11 +105,8 @@ int sq_destroy(sq_ctx *ctx);
 
 int sq_get_info(sq_ctx *ctx, sq_info *info);
 
-/* Whether FP64 passes run in the resident kernel (one node a workgroup, its
- * vectors on chip): planes = the planes of the current vector it keeps in LDS,
- * 0 where the kernel that sq_info reports runs instead (workgroup, batch,
- * gather_trip: the autotuner's choice among the column-marching kernels,
- * which FP32 passes always take). */
+/* Whether FP64 passes run in the resident kernel (sq_info's batch 0): planes = the
+ * planes of the current vector it keeps in LDS, 0 where another kernel runs. */
 int sq_resident_planes(sq_ctx *ctx, int *planes);
 
 /* V_eff on the global grid (npts[0]*npts[1]*npts[2], i fastest), wrapped
@@ -198,7 +197,8 @@ int sq_get_rule_sizes(sq_ctx *ctx, int *n);
  * applies it per precision to its probe times: candidates 0/1 = the one-node
  * kernel with 512/1024 threads, 2/3 = 2 nodes a workgroup with gather trip a/b,
  * 4/5 = 4 nodes with trip a/b (planes a trip: 1/2 in FP64 on the vector ALU;
- * 4 on the matrix cores / 2 on the vector ALU in FP32).  available[6]:
+ * 4 on the matrix cores / 2 on the vector ALU in FP32); FP64 has no 4-node
+ * kernel, 5 is its resident kernel, which SQ_BATCH=0 names.  available[6]:
  * which can launch; probe_ms[6]: their probe times; fixed_* the values of
  * SQ_ZMARCH_WG, SQ_BATCH and SQ_BATCH_TRIP (NULL when unset), which narrow the
  * set.  *candidate = the fastest remaining (lower index on a tie); candidate 0

@@ -69,14 +69,14 @@ struct sq_ctx {
     // the configuration the autotuner chose per precision: nodes per workgroup
     // (1: the one-node z-march kernel in its zwg shape) and gather trip
     int cfg_B[2] = {1, 1}, cfg_ug[2] = {0, 0};
-    float tune_cand[2][6] = {};   // probe ms: one-node 512 / 1024 threads, B=2 trips a/b, B=4 trips a/b
+    float tune_cand[2][6] = {};   // probe ms of the autotuner's candidates (cand_batch)
     // batch list of the last node range
     int2 *batches = nullptr;
     long batch_cap = 0, n_batches = 0, bat_begin = -1, bat_count = -1;
     int bat_B = 0;
     int *probe_ids = nullptr;     // the autotuner's node set (one-node kernel form)
     float *bas32 = nullptr;       // column basis table of the batched kernel's FP32 form
-    // resident kernel (sq_resident.hip): grid (0: not used), planes of v in LDS, dynamic
+    // resident kernel (sq_resident.hip): grid (0: FP64 runs in another kernel), planes of v in LDS, dynamic
     // LDS, images trimmed to the projectors' reach and their padded tables
     int res_grid = 0, res_nl = 0, res_n = 0;
     size_t res_lds = 0, lds_limit = 0;
@@ -773,14 +773,12 @@ static ResParams make_resident_params(const sq_ctx *c, int mode, long begin, lon
 // The resident kernel's tables and shape.  It takes the cubes the column-
 // marching kernels take when their projectors are s+d, no side exceeds its
 // plane limit, no cube meets more images than it holds, and SQ_NO_RESIDENT is
-// not set (SQ_ZMARCH_WG, SQ_BATCH and SQ_BATCH_TRIP choose among the column-
-// marching kernels, which run where this one does not).  Box points past the
-// projectors' reach are dropped: at 2^-53 of the projector's largest value
-// they lie below the rounding of the sums they would enter.
+// not set.  Box points past the projectors' reach are dropped: at 2^-53 of the
+// projector's largest value they lie below the rounding of the sums they would
+// enter.
 static int setup_resident(sq_ctx *c)
 {
     const System &S = c->sys;
-    if (getenv("SQ_NO_RESIDENT")) return SQ_OK;
     const int wg = resident_workgroup(S.nloc);
     if (!c->zmarch || !c->zbatch || wg == 0 || c->img_cap > kResMaxImages) return SQ_OK;
     if (S.ext_points() >= (int64_t)1 << 31 || S.n_nodes() >= (int64_t)1 << 31) return SQ_OK;
@@ -852,15 +850,21 @@ static int launch_resident_pass(sq_ctx *c, int mode, long begin, long count)
     return SQ_OK;
 }
 
-// One Lanczos launch of configuration (B, shape or trip) on the probe's node
-// set, timed by HIP events on the context's stream.
+// One Lanczos launch of configuration (B, shape or trip; B = 0: the resident
+// kernel) on the probe's node set, timed by HIP events on the context's stream.
 static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long nprobe, float *ms)
 {
     hipError_t e = hipSuccess;
     for (int rep = 0; rep < 2; rep++) {   // the first launch loads the code object
         HIP_TRY(hipMemsetAsync(c->queue, 0, 8 * sizeof(int), c->stream));
         HIP_TRY(hipEventRecord(c->ev[0], c->stream));
-        if (B == 1) {
+        if (B == 0) {
+            ResParams P = make_resident_params(c, SQ_NL_KB, 0, nprobe);
+            P.node_list = c->probe_ids;
+            P.nqp = nqp;
+            P.exit_tol = 0;
+            e = launch_resident(P, (int)std::min<long>(c->res_grid, std::max<long>(8, (nprobe + 7) & ~7L)), c->res_lds, c->stream);
+        } else if (B == 1) {
             KParams P = make_params(c, SQ_NL_KB, prec, 0, nprobe, true);
             P.zwg = shape;
             P.node_list = c->probe_ids;
@@ -883,18 +887,27 @@ static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long npr
     return SQ_OK;
 }
 
+// SQ_BATCH of candidate k: the nodes of a workgroup in the column-marching
+// kernels; 0 names the resident kernel, which takes the last place of FP64
+// (the batched kernel with four nodes is built for FP32 alone).
+static int cand_batch(int prec, int k)
+{
+    return k < 2 ? 1 : k < 4 ? 2 : k == 5 && prec == SQ_FP64 ? 0 : 4;
+}
+
 // The autotuner's rule.  Candidates: 0/1 the one-node kernel with 512/1024
-// threads, 2/3 B = 2 with gather trip a/b, 4/5 B = 4 with trip a/b.
-// available[k]: candidate k can launch on this deck.  The environment strings
-// (NULL when unset) narrow the set: SQ_ZMARCH_WG keeps the one-node kernel in
-// that shape, SQ_BATCH the batch size, SQ_BATCH_TRIP the trip of a batched
-// candidate.  Nothing left: candidate 0 when it can launch.
+// threads, 2/3 B = 2 with gather trip a/b, 4/5 B = 4 with trip a/b; in FP64 5 is
+// the resident kernel.  available[k]: candidate k can launch on this deck.  The
+// environment strings (NULL when unset) narrow the set: SQ_ZMARCH_WG keeps the
+// one-node kernel in that shape, SQ_BATCH the batch size (0: the resident
+// kernel), SQ_BATCH_TRIP the trip of a batched candidate.  Nothing left:
+// candidate 0 when it can launch.
 static int tune_allowed(int prec, const int *available, const char *fixed_wg, const char *fixed_b,
                         const char *fixed_t, bool allow[6])
 {
     int n = 0;
     for (int k = 0; k < 6; k++) {
-        const int B = k < 2 ? 1 : (k < 4 ? 2 : 4);
+        const int B = cand_batch(prec, k);
         allow[k] = available[k] != 0;
         if (fixed_wg) allow[k] = B == 1 && (atoi(fixed_wg) == 1024) == (k == 1) && available[k];
         if (fixed_b && atoi(fixed_b) != B) allow[k] = false;
@@ -925,10 +938,11 @@ static int tune_pick(const bool allow[6], const float ms[6])
 // runs fewer) -- and keeps the fastest:
 //   the one-node z-march kernel with 512 threads (two columns a thread) or
 //   1024 (one); the batched kernel with B = 2 (FP64, FP32) or 4 (FP32) nodes
-//   a workgroup, each with two gather trips.
+//   a workgroup, each with two gather trips; the resident kernel (FP64).
 // The same nodes and steps for every candidate, so the times compare
 // directly.  SQ_ZMARCH_WG=512|1024 fixes the one-node kernel in that shape;
-// SQ_BATCH=1|2|4 (and SQ_BATCH_TRIP) fixes the batch size (and trip).
+// SQ_BATCH=1|2|4 (and SQ_BATCH_TRIP) fixes the batch size (and trip), SQ_BATCH=0
+// the resident kernel; SQ_NO_RESIDENT leaves that one out.
 int finish_device_setup(sq_ctx *c)
 {
     const System &S = c->sys;
@@ -955,7 +969,14 @@ int finish_device_setup(sq_ctx *c)
                     scratch = std::max(scratch, (size_t)g * 3 * (S.nloc[2] + B - 1) * ncol * B * el);
                 }
     }
-    if (int rc = setup_resident(c)) return rc;
+    const char *fixed_wg = getenv("SQ_ZMARCH_WG");
+    const char *fixed_b = getenv("SQ_BATCH");
+    const char *fixed_t = getenv("SQ_BATCH_TRIP");
+    const int all[6] = {1, 1, 1, 1, 0, 1};
+    bool may[6];
+    tune_allowed(SQ_FP64, all, fixed_wg, fixed_b, fixed_t, may);
+    if (may[5] && !getenv("SQ_NO_RESIDENT"))
+        if (int rc = setup_resident(c)) return rc;
     scratch = std::max(scratch, (size_t)c->res_grid * (S.nloc[2] - c->res_nl) * S.nloc[0] * S.nloc[1] * sizeof(double));
     HIP_TRY(hipMalloc(&c->scratch, scratch));
     if (!c->zmarch) return SQ_OK;
@@ -965,9 +986,6 @@ int finish_device_setup(sq_ctx *c)
         c->cfg_B[prec] = 1;
         c->cfg_ug[prec] = 0;
     }
-    const char *fixed_wg = getenv("SQ_ZMARCH_WG");
-    const char *fixed_b = getenv("SQ_BATCH");
-    const char *fixed_t = getenv("SQ_BATCH_TRIP");
     // the probe's node set
     const int lz = S.box[5];
     const long plane = (long)S.box[3] * S.box[4];
@@ -987,16 +1005,17 @@ int finish_device_setup(sq_ctx *c)
     for (int prec = 0; prec < 2; prec++) {
         int available[6];
         for (int k = 0; k < 6; k++) {
-            const int B = k < 2 ? 1 : (k < 4 ? 2 : 4);
-            available[k] = B == 1 ? grids[prec][k] > 0
-                                  : (c->zbatch && zbatch_grid(c, prec, B, batch_trip(prec, k & 1)) > 0);
+            const int B = cand_batch(prec, k);
+            available[k] = B == 0   ? c->res_grid > 0
+                           : B == 1 ? grids[prec][k] > 0
+                                    : (c->zbatch && zbatch_grid(c, prec, B, batch_trip(prec, k & 1)) > 0);
         }
         bool allow[6];
         const int n_allowed = tune_allowed(prec, available, fixed_wg, fixed_b, fixed_t, allow);
         float ms[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < 6 && n_allowed > 1; k++) {
             if (!allow[k]) continue;
-            const int B = k < 2 ? 1 : (k < 4 ? 2 : 4);
+            const int B = cand_batch(prec, k);
             if (B > 1 && (rc = upload_batches(c, bl[B]))) return rc;
             if ((rc = probe_launch(c, prec, B, B == 1 ? (k ? 1024 : 512) : batch_trip(prec, k & 1), nqp, (long)ids.size(),
                                    &ms[k])))
@@ -1006,11 +1025,18 @@ int finish_device_setup(sq_ctx *c)
         }
         int best = tune_pick(allow, ms);
         if (best < 0) best = 0;
-        if (best < 2) {
+        const int B = cand_batch(prec, best);
+        if (B && prec == SQ_FP64 && c->res_grid) {   // another kernel: the resident one's tables go
+            (void)hipFree(c->res_tab);
+            (void)hipFree(c->res_img);
+            c->res_tab = nullptr;
+            c->res_img = nullptr;
+            c->res_grid = 0;
+        }
+        if (B == 1) {
             c->zwg[prec] = best ? 1024 : 512;
             c->zgrid[prec] = grids[prec][best];
-        } else {
-            const int B = best < 4 ? 2 : 4;
+        } else if (B > 1) {
             c->cfg_B[prec] = B;
             c->cfg_ug[prec] = batch_trip(prec, best & 1);
             // the one-node kernel stays available (force pass, node lists) in the 1024 shape when it fits
@@ -1142,10 +1168,11 @@ int sq_get_info(sq_ctx *c, sq_info *I)
     I->kernel = c->zmarch ? 1 : 0;
     I->kmax = c->kmax;
     for (int prec = 0; prec < 2; prec++) {
-        I->workgroup[prec] = c->zmarch ? (c->cfg_B[prec] > 1 ? 1024 : c->zwg[prec]) : 1024;
+        const bool resident = prec == SQ_FP64 && c->res_grid;
+        I->workgroup[prec] = resident ? resident_workgroup(S.nloc) : c->zmarch ? (c->cfg_B[prec] > 1 ? 1024 : c->zwg[prec]) : 1024;
         I->tune_ms[prec][0] = c->tune_ms[prec][0];
         I->tune_ms[prec][1] = c->tune_ms[prec][1];
-        I->batch[prec] = c->zmarch ? c->cfg_B[prec] : 1;
+        I->batch[prec] = resident ? 0 : c->zmarch ? c->cfg_B[prec] : 1;
         I->gather_trip[prec] = c->cfg_ug[prec];
         for (int k = 0; k < 6; k++) I->tune_candidates_ms[prec][k] = c->tune_cand[prec][k];
     }
