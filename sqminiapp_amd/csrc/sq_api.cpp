@@ -102,7 +102,7 @@ struct sq_ctx {
     double *c64 = nullptr;  // 3 x (kMaxOrder+1)
     float *c32 = nullptr;
     void *scratch = nullptr;
-    double *a = nullptr, *b = nullptr, *lam = nullptr, *w = nullptr, *lmin = nullptr, *lmax = nullptr;
+    double *a = nullptr, *b = nullptr, *lam = nullptr, *w = nullptr, *lmin = nullptr, *lmax = nullptr, *qlws = nullptr;
     int *status = nullptr;
     int *queue = nullptr, *nsteps = nullptr;   // z-march work queue (8 counters); Gauss nodes per node
     double *partial = nullptr, *out = nullptr;
@@ -160,7 +160,7 @@ void free_ctx(sq_ctx *c)
     if (!c) return;
     void *ptrs[] = {c->img_dimp, c->rad64, c->rad32, c->img_rad, c->img_cen, c->chi64, c->chi32, c->img_lo, c->img_dim, c->img_off, c->img_atom, c->img_type, c->gamma,
                     c->cov_off, c->cov_img, c->diag64, c->diag32, c->c64, c->c32, c->scratch, c->a, c->b,
-                    c->lam, c->w, c->lmin, c->lmax, c->status, c->partial, c->bis, c->out,
+                    c->lam, c->w, c->lmin, c->lmax, c->qlws, c->status, c->partial, c->bis, c->out,
                     c->queue, c->nsteps, c->batches, c->probe_ids, c->bas32, c->res_img,
                     c->res_tab};
     void *scf_ptrs[] = {c->scf.rho, c->scf.rho_out, c->scf.b, c->scf.phi, c->scf.eps, c->scf.vxc, c->scf.veff, c->scf.r,
@@ -424,6 +424,7 @@ int create_device(sq_ctx *c, int device)
     HIP_TRY(hipMalloc((void **)&c->lmin, nn * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->lmax, nn * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->status, std::max<int64_t>(nn, 1) * sizeof(int)));
+    if (const size_t q = ql_workspace_bytes(S.nqp, nn)) HIP_TRY(hipMalloc((void **)&c->qlws, q));
     HIP_TRY(hipMalloc((void **)&c->partial, 3 * kRedBlocks * sizeof(double)));
     HIP_TRY(hipMalloc((void **)&c->bis, 2 * sizeof(BisState)));
     HIP_TRY(hipMalloc((void **)&c->out, 4 * sizeof(double)));
@@ -1239,7 +1240,7 @@ int sq_run(sq_ctx *c, int mode, int precision, long begin, long count)
     HIP_TRY(hipEventRecord(c->ev[2], c->stream));
     HIP_TRY(launch_ql(c->a + begin * (S.nqp + 1), c->b + begin * (S.nqp + 1), S.nqp, S.nqp + 1, count,
                       c->lam + begin * S.nqp, c->w + begin * S.nqp, c->lmin + begin, c->lmax + begin, c->status + begin,
-                      c->stream, c->last_exit ? c->nsteps + begin : nullptr));
+                      c->qlws, c->stream, c->last_exit ? c->nsteps + begin : nullptr));
     HIP_TRY(hipEventRecord(c->ev[3], c->stream));
     HIP_TRY(hipEventSynchronize(c->ev[3]));
     if ((rc = check_status(c, begin, count, "QL"))) return rc;
@@ -1354,14 +1355,14 @@ int sq_tridiag_nodes_weights(sq_ctx *c, const double *diag, const double *subdia
     const size_t m = (size_t)n * count;
     double *buf = nullptr;
     int *st = nullptr;
-    HIP_TRY(hipMalloc((void **)&buf, (2 * m + 2 * m + 2 * count) * sizeof(double)));
+    HIP_TRY(hipMalloc((void **)&buf, (2 * m + 2 * m + 2 * count) * sizeof(double) + ql_workspace_bytes(n, count)));
     hipError_t e = hipMalloc((void **)&st, count * sizeof(int));
     if (e != hipSuccess) { (void)hipFree(buf); return set_err(SQ_ERR_DEVICE, "hipMalloc failed"); }
-    double *da = buf, *db = da + m, *dl = db + m, *dw = dl + m, *dmin = dw + m, *dmax = dmin + count;
+    double *da = buf, *db = da + m, *dl = db + m, *dw = dl + m, *dmin = dw + m, *dmax = dmin + count, *ws = dmax + count;
     int rc = SQ_OK;
     if (hipMemcpy(da, diag, m * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(db, subdiag, m * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        launch_ql(da, db, n, n, count, dl, dw, dmin, dmax, st, c->stream) != hipSuccess ||
+        launch_ql(da, db, n, n, count, dl, dw, dmin, dmax, st, ws, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         rc = set_err(SQ_ERR_DEVICE, "QL device step failed");
     if (!rc) {
@@ -1828,7 +1829,7 @@ static int enqueue_sq_pass(sq_ctx *c, int mode, int precision)
         HIP_TRY(launch_lanczos(P, precision, (int)std::min<long>(c->grid, count), c->lds, st));
     }
     HIP_TRY(launch_status_any(c->status, count, c->scf.ctl, st));
-    HIP_TRY(launch_ql(c->a, c->b, S.nqp, S.nqp + 1, count, c->lam, c->w, c->lmin, c->lmax, c->status, st,
+    HIP_TRY(launch_ql(c->a, c->b, S.nqp, S.nqp + 1, count, c->lam, c->w, c->lmin, c->lmax, c->status, c->qlws, st,
                       c->last_exit ? c->nsteps : nullptr));
     HIP_TRY(launch_status_any(c->status, count, c->scf.ctl, st));
     return SQ_OK;

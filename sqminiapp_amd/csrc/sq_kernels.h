@@ -83,8 +83,10 @@ hipError_t launch_basis_tables(const double *rad, int n_images, const int4 *lo, 
                                const double4 *cen, double hz, double rz, float *b32, hipStream_t st);
 hipError_t launch_apply(const KParams &P, long id, const double *x, double *y, int nonlocal_only, size_t lds,
                         hipStream_t st);
+// QL of count tridiagonals; ws: ql_workspace_bytes(n, count), which does not fall as count grows
+size_t ql_workspace_bytes(int n, long count);
 hipError_t launch_ql(const double *a, const double *b, int n, int stride, long count, double *lam, double *w,
-                     double *lmin, double *lmax, int *status, hipStream_t st, const int *nsteps = nullptr);
+                     double *lmin, double *lmax, int *status, double *ws, hipStream_t st, const int *nsteps = nullptr);
 // QL of host-supplied device tridiagonals with its workspace in the library's
 // static device array (no allocation): the array's per-device address
 // (noalloc_scratch_init, with the device current), the bytes a call needs, and

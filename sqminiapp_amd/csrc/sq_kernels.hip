@@ -256,28 +256,27 @@ __device__ __forceinline__ void rotation(double f, double g, double &r, double &
 //
 // Bound by the chain of one rotation (rotation(), about 400
 // clocks) times the rotations of a tridiagonal (5000 at n = 80), so what counts
-// is that nothing else joins the chain: d, e and z lie in LDS as [i][lane], the
-// next rotation's entries are read ahead, and the test for a small
+// is that nothing else joins the chain and that many chains run side by side.
+// The next rotation's entries are read ahead, and the test for a small
 // off-diagonal, which the reference repeats from l on after every sweep, is
-// made inside the sweep, where d and e become final.  Only `lanes` lanes of a
-// wavefront work, so that a batch spreads over all SIMDs and few tridiagonals
-// wait for each other's sweeps.  16384 x n = 80: 3.1 ms; 11.4 with the three rows
-// in device memory and a scan before each sweep, 3.3 with the operators in place
-// of rotation().
-__global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, const double *__restrict__ bsub, int nmax,
-                                                int stride, long count, int lanes, double *__restrict__ lam,
-                                                double *__restrict__ w, double *__restrict__ lmin,
-                                                double *__restrict__ lmax, int *__restrict__ status,
-                                                const int *__restrict__ nsteps)
+// made inside the sweep, where d and e become final; a scan before each sweep
+// and the operators in place of rotation() took 13.3 ms for 16384 x n = 80, which
+// take 3.8 now.  The rows d, e and z lie in LDS (ql_kernel) or, for batches of which
+// LDS holds only a part at a time, in device memory (ql_kernel_mem); ql_lanes.
+
+// Tridiagonals t0 .. t0 + mine - 1, one a lane; d, e and z of lane k at
+// rows[i * pitch + k], i in [0, nmax), [nmax, 2 nmax) and [2 nmax, 3 nmax).  The
+// outputs may be the inputs: a tridiagonal is read before any is written.
+__device__ __forceinline__ void ql_rules(double *rows, const unsigned pitch, const double *a, const double *bsub, int nmax,
+                                         int stride, long t0, int mine, double *lam, double *w, double *lmin, double *lmax,
+                                         int *status, const int *nsteps)
 {
-    extern __shared__ double rows[];   // d, e, z: [3][nmax][lanes]
-    const long t0 = (long)blockIdx.x * lanes;
-    const int mine = (int)min((long)lanes, count - t0), lane = threadIdx.x;
+    const int lane = threadIdx.x;
     for (int q = lane; q < mine * nmax; q += 64) {
         const int k = q / nmax, i = q - k * nmax;
-        rows[i * lanes + k] = a[(t0 + k) * stride + i];
-        rows[(nmax + i) * lanes + k] = bsub[(t0 + k) * stride + i];
-        rows[(2 * nmax + i) * lanes + k] = i == 0 ? 1.0 : 0.0;
+        rows[i * pitch + k] = a[(t0 + k) * stride + i];
+        rows[(nmax + i) * pitch + k] = bsub[(t0 + k) * stride + i];
+        rows[(2 * nmax + i) * pitch + k] = i == 0 ? 1.0 : 0.0;
     }
     __syncthreads();
     const long t = t0 + lane;
@@ -286,10 +285,10 @@ __global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, co
     int n = nmax, bad = 0;
     if (lane < mine) {
         if (nsteps) n = max(1, min(nmax, nsteps[t]));
-        double *const d = rows + lane, *const e = rows + nmax * lanes + lane, *const z = rows + 2 * nmax * lanes + lane;
-#define D(i) d[(i) * lanes]
-#define EE(i) e[(i) * lanes]
-#define Z(i) z[(i) * lanes]
+        double *const d = rows + lane, *const e = rows + nmax * pitch + lane, *const z = rows + 2 * nmax * pitch + lane;
+#define D(i) d[(unsigned)(i) * pitch]
+#define EE(i) e[(unsigned)(i) * pitch]
+#define Z(i) z[(unsigned)(i) * pitch]
         EE(n - 1) = 0.0;
         auto small = [](double ei, double di, double dn) {
             const double dd = fabs(di) + fabs(dn);
@@ -383,9 +382,33 @@ __global__ void __launch_bounds__(64) ql_kernel(const double *__restrict__ a, co
     for (int q = lane; q < mine * nmax; q += 64) {
         const int k = q / nmax, i = q - k * nmax;
         if (failed >> k & 1) continue;
-        const double zi = rows[(2 * nmax + i) * lanes + k];
-        lam[(t0 + k) * nmax + i] = rows[i * lanes + k];
+        const double zi = rows[(2 * nmax + i) * pitch + k];
+        lam[(t0 + k) * nmax + i] = rows[i * pitch + k];
         w[(t0 + k) * nmax + i] = zi * zi;
+    }
+}
+
+// Rows in LDS; only `lanes` lanes of a wavefront work, so that a batch spreads over
+// all SIMDs and few tridiagonals wait for each other's sweeps.
+__global__ void __launch_bounds__(64) ql_kernel(const double *a, const double *bsub, int nmax, int stride, long count,
+                                                int lanes, double *lam, double *w, double *lmin, double *lmax, int *status,
+                                                const int *nsteps)
+{
+    extern __shared__ double rows[];   // d, e, z: [3][nmax][lanes]
+    const long t0 = (long)blockIdx.x * lanes;
+    ql_rules(rows, lanes, a, bsub, nmax, stride, t0, (int)min((long)lanes, count - t0), lam, w, lmin, lmax, status, nsteps);
+}
+
+// Rows in device memory, 3 nmax x pitch doubles at ws: 64 tridiagonals a wavefront, and
+// the wavefront's next ones in the same place.
+__global__ void __launch_bounds__(64) ql_kernel_mem(const double *a, const double *bsub, int nmax, int stride, long count,
+                                                    unsigned pitch, double *ws, double *lam, double *w, double *lmin,
+                                                    double *lmax, int *status, const int *nsteps)
+{
+    double *const rows = ws + blockIdx.x * 64u;
+    for (long t0 = blockIdx.x * 64L; t0 < count; t0 += gridDim.x * 64L) {
+        ql_rules(rows, pitch, a, bsub, nmax, stride, t0, (int)min(64L, count - t0), lam, w, lmin, lmax, status, nsteps);
+        __syncthreads();
     }
 }
 
@@ -585,26 +608,43 @@ hipError_t launch_apply(const KParams &P, long id, const double *x, double *y, i
     return hipGetLastError();
 }
 
-// Tridiagonals a wavefront of ql_kernel takes: the fewest with which every
-// wavefront has a CU to itself (n = 80: 33 take 2.6 ms one a wavefront and 2.9
-// sixteen a wavefront; 3840 take 3.65 sixteen a wavefront and 4.4 eight; 7872
-// take 3.9 and 4.7 with 32 and 16), else 16 on four wavefronts a CU (16384:
-// 3.1, against 3.6 with 32), as far as their rows fit LDS.
+// Tridiagonals a wavefront of ql_kernel takes, 0: ql_kernel_mem.  LDS while the
+// batch runs in one round: the fewest lanes with which every wavefront has a CU to
+// itself (n = 80: 33 take 2.8 ms one a wavefront and 3.8 sixteen a wavefront; 4096
+// take 4.6 sixteen a wavefront and 5.4 eight), else 16 on four wavefronts a CU
+// (16384: 3.8, against 4.3 with 32).  Past that device memory, whose latency
+// other wavefronts hide (LDS form, memory form; n = 80: 16384 take 3.8 and 4.6 ms,
+// 20000 9.3 and 5.4, 200000 51 and 22; n = 256: 1024 take 36 and 41, 4096 71 and 48,
+// 24576 329 and 60).
 static int ql_lanes(int n, long count)
 {
     const size_t row = (size_t)3 * n * sizeof(double);
     int lanes = 1;
     while (lanes < 32 && (count + lanes - 1) / lanes > 256) lanes <<= 1;
-    if ((count + lanes - 1) / lanes > 256) lanes = 16;
-    while (lanes > 1 && lanes * row > (lanes > 16 ? 65536 : 40960)) lanes >>= 1;
-    return lanes;
+    if ((count + lanes - 1) / lanes <= 256 && lanes * row <= 65536) return lanes;
+    return (count + 15) / 16 <= 1024 && 16 * row <= 40960 ? 16 : 0;
+}
+
+// Wavefronts of ql_kernel_mem: up to eight a CU, the batch in rounds past that
+static long ql_mem_grid(long count) { return std::min<long>((count + 63) / 64, 2048); }
+
+size_t ql_workspace_bytes(int n, long count)
+{
+    return ql_lanes(n, count) ? 0 : (size_t)3 * n * std::min(count, 64 * ql_mem_grid(count)) * sizeof(double);
 }
 
 hipError_t launch_ql(const double *a, const double *b, int n, int stride, long count, double *lam, double *w,
-                     double *lmin, double *lmax, int *status, hipStream_t st, const int *nsteps)
+                     double *lmin, double *lmax, int *status, double *ws, hipStream_t st, const int *nsteps)
 {
     if (n < 1 || n > kMaxNqp || count <= 0) return hipErrorInvalidValue;
     const int lanes = ql_lanes(n, count);
+    if (lanes == 0) {
+        if (!ws) return hipErrorInvalidValue;
+        const long grid = ql_mem_grid(count);
+        hipLaunchKernelGGL(ql_kernel_mem, dim3((unsigned)grid), dim3(64), 0, st, a, b, n, stride, count,
+                           (unsigned)std::min(count, 64 * grid), ws, lam, w, lmin, lmax, status, nsteps);
+        return hipGetLastError();
+    }
     const long blocks = (count + lanes - 1) / lanes;
     // LDS for the rows, and no less than keeps a CU from taking more workgroups than its share
     const size_t rows = (size_t)lanes * 3 * n * sizeof(double);
@@ -676,9 +716,8 @@ void *noalloc_scratch(int device)
     return g_scratch_dev[device];
 }
 
-// workspace layout: [3][n][count] doubles, the room of QL's three rows in device
-// memory (it keeps them in LDS now; the limit on a batch is the interface's) |
-// status[count] | the index of the first failed tridiagonal (long long)
+// workspace layout: [3][n][count] doubles, the rows of ql_kernel_mem (which never
+// takes more) | status[count] | the index of the first failed tridiagonal (long long)
 size_t noalloc_ql_bytes(int n, long count)
 {
     return align256((size_t)3 * n * count * sizeof(double)) + align256((size_t)count * sizeof(int)) + 256;
@@ -710,7 +749,7 @@ hipError_t launch_ql_noalloc(void *ws, const double *a, const double *b, int n, 
     int *status = reinterpret_cast<int *>(base + align256((size_t)3 * n * count * sizeof(double)));
     long long *bad = reinterpret_cast<long long *>(reinterpret_cast<unsigned char *>(status) +
                                                    align256((size_t)count * sizeof(int)));
-    hipError_t e = launch_ql(a, b, n, n, count, lam, w, lmin, lmax, status, st);
+    hipError_t e = launch_ql(a, b, n, n, count, lam, w, lmin, lmax, status, static_cast<double *>(ws), st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(first_failure, dim3(1), dim3(256), 0, st, status, count, bad);
     *first_bad = bad;
