@@ -2379,14 +2379,25 @@ struct DevBufs {
 // Pieces of a model's workspace, each 256-byte aligned, while its lock is held.  It
 // grows to what a pass needs and stays, up to kMlpKeep, until the model is destroyed:
 // an allocation and a release of each piece cost a call more than its kernels.
+// A pass ends with finish(); one that fails on the way still waits for what it queued
+// before the lock goes and before its callers' buffers do.
 constexpr size_t kMlpKeep = 256u << 20;
 struct MlpSpace {
     sq_mlp *m;
+    hipStream_t st;   // the pass's
     std::lock_guard<std::mutex> hold;
     size_t used = 0;
-    explicit MlpSpace(sq_mlp *m_) : m(m_), hold(m_->ws_lock) {}
+    bool idle = false;
+    MlpSpace(sq_mlp *m_, hipStream_t st_) : m(m_), st(st_), hold(m_->ws_lock) {}
+    int finish()
+    {
+        HIP_TRY(hipStreamSynchronize(st));
+        idle = true;
+        return SQ_OK;
+    }
     ~MlpSpace()
     {
+        if (!idle) (void)hipStreamSynchronize(st);
         if (m->ws_bytes <= kMlpKeep) return;
         (void)hipFree(m->ws);
         m->ws = nullptr;
@@ -2606,14 +2617,13 @@ int sq_mlp_loss_grad(sq_mlp *m, const float *X, const float *T, long N, double *
 {
     if (!m || !X || !T || N <= 0) return set_err(SQ_ERR_ARG, "bad argument");
     HIP_TRY(hipSetDevice(m->device));
-    MlpSpace space(m);
+    MlpSpace space(m, m->stream);
     MlpScratch W;
     int rc;
     if ((rc = W.alloc(space, m, N))) return rc;
     HIP_TRY(hipMemcpy(W.X, X, N * m->K * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(W.T, T, N * sizeof(float), hipMemcpyHostToDevice));
-    if ((rc = mlp_loss_grad_dev(m, N, loss, W))) return rc;
-    HIP_TRY(hipStreamSynchronize(m->stream));
+    if ((rc = mlp_loss_grad_dev(m, N, loss, W)) || (rc = space.finish())) return rc;
     if (grad) HIP_TRY(hipMemcpy(grad, m->g, m->np * sizeof(double), hipMemcpyDeviceToHost));
     return SQ_OK;
 }
@@ -2630,7 +2640,7 @@ int sq_mlp_forward(sq_mlp *m, const float *X, long N, int bf16, int normalize, f
 {
     if (!m || !X || !Y || N <= 0) return set_err(SQ_ERR_ARG, "bad argument");
     HIP_TRY(hipSetDevice(m->device));
-    MlpSpace space(m);
+    MlpSpace space(m, m->stream);
     const size_t rows = N;
     int rc;
     if ((rc = space.reserve(space.piece(rows * m->K * 4) + space.piece(rows * 4) + space.piece(2 * m->K * 4)))) return rc;
@@ -2640,8 +2650,7 @@ int sq_mlp_forward(sq_mlp *m, const float *X, long N, int bf16, int normalize, f
     HIP_TRY(launch_mlp_forward(dX, N, m->p, normalize ? norm : nullptr, normalize ? norm + m->K : nullptr, nullptr, nullptr,
                                nullptr, nullptr, dY, bf16, m->stream));
     HIP_TRY(hipMemcpyAsync(Y, dY, N * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipStreamSynchronize(m->stream));
-    return SQ_OK;
+    return space.finish();
 }
 
 int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
@@ -2669,7 +2678,7 @@ int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
         for (int q = 0; q < K; q++) Xn[n * K + q] = (m->X[n * K + q] - m->mean[q]) * m->rstd[q];
         Tn[n] = (float)(m->T[n] / m->tscale);
     }
-    MlpSpace space(m);
+    MlpSpace space(m, m->stream);
     MlpScratch W;
     int rc;
     if ((rc = W.alloc(space, m, N))) return rc;
@@ -2681,8 +2690,7 @@ int sq_mlp_train(sq_mlp *m, int epochs, double lr, double *loss)
         if ((e & 63) == 63) HIP_TRY(hipStreamSynchronize(m->stream));
     }
     if (loss && (rc = mlp_loss_grad_dev(m, N, loss, W))) return rc;
-    HIP_TRY(hipStreamSynchronize(m->stream));
-    return SQ_OK;
+    return space.finish();
 }
 
 // The guess where model and context share a device: descriptors, network, superposed atoms and
@@ -2702,8 +2710,10 @@ static int mlp_guess_dev(sq_mlp *m, sq_ctx *c, const int G[3], int bf16, double 
         tab.insert(tab.end(), P.s_uu.yd.begin(), P.s_uu.yd.end());
     }
     HIP_TRY(hipSetDevice(m->device));
-    MlpSpace W(m);
     int rc, flags[2];
+    double tot;
+    hipStream_t st = c->stream;
+    MlpSpace W(m, st);
     if ((rc = W.reserve(W.piece(ng * kMlpK * 4) + W.piece(ng * 4) + W.piece(2 * kMlpK * 4) + W.piece(img.size() * sizeof(double4)) +
                         W.piece(sizeof flags) + W.piece(ng * 8) + W.piece(kRedBlocks * 8) + W.piece(2 * 8) +
                         W.piece(dimg.size() * sizeof(DensityImage)) + W.piece(types.size() * sizeof(DensityType)) +
@@ -2716,7 +2726,6 @@ static int mlp_guess_dev(sq_mlp *m, sq_ctx *c, const int G[3], int bf16, double 
     DensityImage *const rimg = W.get<DensityImage>(dimg.size());
     DensityType *const rtypes = W.get<DensityType>(types.size());
     double *const rtab = W.get<double>(tab.size());
-    hipStream_t st = c->stream;
     if ((rc = mlp_put_norm(m, norm))) return rc;
     HIP_TRY(hipMemcpyAsync(ximg, img.data(), img.size() * sizeof(double4), hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(rimg, dimg.data(), dimg.size() * sizeof(DensityImage), hipMemcpyHostToDevice, st));
@@ -2731,10 +2740,9 @@ static int mlp_guess_dev(sq_mlp *m, sq_ctx *c, const int G[3], int bf16, double 
     HIP_TRY(launch_guess_add(rho, Y, sums, (double)S.noetot, S.dV, m->tscale, (long)ng, st));
     HIP_TRY(launch_dot(rho, nullptr, (long)ng, 1.0, part, kRedBlocks, sums + 1, st));
     HIP_TRY(launch_guess_scale(rho, sums + 1, (double)S.noetot, S.dV, (long)ng, st));
-    double tot;
     HIP_TRY(hipMemcpyAsync(flags, xflags, sizeof flags, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(&tot, sums + 1, sizeof tot, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    if ((rc = W.finish())) return rc;
     if (flags[0]) return set_err(SQ_ERR_RANGE, "descriptors: more atoms within the cutoff of a point than the kernel holds");
     if (flags[1]) return set_err(flags[1], "atomic density: spline evaluation failed");
     if (!(tot * S.dV > 0)) return set_err(SQ_ERR_RANGE, "network density has no charge");
