@@ -853,10 +853,12 @@ static int launch_resident_pass(sq_ctx *c, int mode, long begin, long count)
 
 // One Lanczos launch of configuration (B, shape or trip; B = 0: the resident
 // kernel) on the probe's node set, timed by HIP events on the context's stream.
-static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long nprobe, float *ms)
+// The launch before it loads the code object: on `warm` nodes.
+static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long all, long warm, float *ms)
 {
     hipError_t e = hipSuccess;
-    for (int rep = 0; rep < 2; rep++) {   // the first launch loads the code object
+    for (int rep = 0; rep < 2; rep++) {
+        const long nprobe = rep ? all : std::min(warm, all);
         HIP_TRY(hipMemsetAsync(c->queue, 0, 8 * sizeof(int), c->stream));
         HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         if (B == 0) {
@@ -874,10 +876,11 @@ static int probe_launch(sq_ctx *c, int prec, int B, int shape, int nqp, long npr
             const int grid = (int)std::min<long>(zmarch_grid(c, prec, shape), std::max<long>(8, (nprobe + 7) & ~7L));
             e = launch_zmarch(P, prec, grid, c->zlds, c->stream);
         } else {
-            KParams P = make_batch_params(c, SQ_NL_KB, prec, B, c->batches, c->n_batches);
+            const long n = std::min(c->n_batches, nprobe);
+            KParams P = make_batch_params(c, SQ_NL_KB, prec, B, c->batches, n);
             P.nqp = nqp;
             P.exit_tol = 0;
-            const int grid = (int)std::min<long>(c->zb_grid[prec][B], std::max<long>(8, (c->n_batches + 7) & ~7L));
+            const int grid = (int)std::min<long>(c->zb_grid[prec][B], std::max<long>(8, (n + 7) & ~7L));
             e = launch_zbatch(P, prec, B, shape, grid, c->zb_lds[B], c->stream);
         }
         if (e != hipSuccess) return set_err(SQ_ERR_DEVICE, std::string("autotuner probe: ") + hipGetErrorString(e));
@@ -1014,12 +1017,15 @@ int finish_device_setup(sq_ctx *c)
         bool allow[6];
         const int n_allowed = tune_allowed(prec, available, fixed_wg, fixed_b, fixed_t, allow);
         float ms[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        // candidates within a few per cent of each other are timed after a whole launch;
+        // the resident kernel leads by half and more, so a few nodes do beside it
+        const long warm = available[5] && prec == SQ_FP64 ? 8 : (long)ids.size();
         for (int k = 0; k < 6 && n_allowed > 1; k++) {
             if (!allow[k]) continue;
             const int B = cand_batch(prec, k);
             if (B > 1 && (rc = upload_batches(c, bl[B]))) return rc;
             if ((rc = probe_launch(c, prec, B, B == 1 ? (k ? 1024 : 512) : batch_trip(prec, k & 1), nqp, (long)ids.size(),
-                                   &ms[k])))
+                                   warm, &ms[k])))
                 return rc;
             c->tune_cand[prec][k] = ms[k];
             if (k < 2) c->tune_ms[prec][k] = ms[k];
