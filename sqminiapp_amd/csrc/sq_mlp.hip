@@ -141,8 +141,12 @@ __global__ void __launch_bounds__(256) mlp_features(const double4 *__restrict__ 
 
 // A point a thread, a brick of points a block, which lists in order the images whose box
 // meets the brick.  A point's sum runs over its images in order, so it is the host's
-// (build_atomic_density), bit for bit.  The cell of 128 atoms
-// takes 73 us, and 3 ms on 16 host threads.
+// (build_atomic_density), bit for bit.  Bound by the bisection's chain of loads, the more
+// the fewer bricks a cell has, so four images' bisections run side by side (two bricks
+// of 108 points: 0.58 ms, 0.67 one after the other; 660 points: 0.18 and 0.25).  The
+// cell of 128 atoms takes 72 us, and 3 ms on 16 host threads.
+constexpr int kBeside = 4;
+
 __global__ void __launch_bounds__(256) superposed_density(const DensityImage *__restrict__ img, int nimg,
                                                           const DensityType *__restrict__ types,
                                                           const double *__restrict__ tab, int G0, int G1, int G2, double h0,
@@ -176,17 +180,42 @@ __global__ void __launch_bounds__(256) superposed_density(const DensityImage *__
         __syncthreads();
         if (listed <= kCand - 256 && base + 256 < nimg) continue;   // room for the next 256
         if (inside)
-            for (int a = 0; a < listed; a++) {
-                const DensityImage &im = img[list[a]];
-                if (i < im.lo[0] || i > im.hi[0] || j < im.lo[1] || j > im.hi[1] || k < im.lo[2] || k > im.hi[2]) continue;
-                const DensityType T = types[im.at];
-                const double *x = tab + T.off;
-                const double dx = h0 * i - R0 - im.X[0], dy = h1 * j - R1 - im.X[1], dz = h2 * k - R2 - im.X[2];
-                const double r = sqrt(dx * dx + dy * dy + dz * dz);
-                if (!(r <= x[T.n - 1])) continue;
-                double v;
-                if (!spline_at(x, x + T.n, x + 2 * T.n, T.n, r, &v)) { *status = 3; continue; }
-                sum += v;
+            for (int a = 0; a < listed; a += kBeside) {
+                const double *x[kBeside];
+                double r[kBeside];
+                int n[kBeside], lo[kBeside], hi[kBeside];   // bisection: lower_bound; n = 0: nothing to add
+#pragma unroll
+                for (int u = 0; u < kBeside; u++) {
+                    const DensityImage &im = img[list[min(a + u, listed - 1)]];
+                    const DensityType T = types[im.at];
+                    x[u] = tab + T.off;
+                    const double dx = h0 * i - R0 - im.X[0], dy = h1 * j - R1 - im.X[1], dz = h2 * k - R2 - im.X[2];
+                    r[u] = sqrt(dx * dx + dy * dy + dz * dz);
+                    const bool in = a + u < listed && i >= im.lo[0] && i <= im.hi[0] && j >= im.lo[1] && j <= im.hi[1] &&
+                                    k >= im.lo[2] && k <= im.hi[2] && r[u] <= x[u][T.n - 1];
+                    if (in && !(r[u] >= x[u][0])) *status = 3;
+                    n[u] = in && r[u] >= x[u][0] ? T.n : 0;
+                    lo[u] = 0;
+                    hi[u] = n[u];
+                }
+                for (bool more = true; more;) {
+                    more = false;
+#pragma unroll
+                    for (int u = 0; u < kBeside; u++) {
+                        const int mid = (lo[u] + hi[u]) >> 1;
+                        const bool open = lo[u] < hi[u], less = x[u][mid] < r[u];   // x[0] of a closed one without knots
+                        lo[u] = open && less ? mid + 1 : lo[u];
+                        hi[u] = open && !less ? mid : hi[u];
+                        more = more || lo[u] < hi[u];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kBeside; u++)
+                    if (n[u]) {
+                        double v;
+                        spline_cubic(x[u], x[u] + n[u], x[u] + 2 * n[u], n[u], lo[u], r[u], &v);
+                        sum += v;
+                    }
             }
         listed = 0;
         __syncthreads();

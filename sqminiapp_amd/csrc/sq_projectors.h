@@ -22,20 +22,12 @@ struct TabType {
 // Returns 0, or 4 when a type has more than 16 channels.
 int pack_projector_splines(const System &S, std::vector<double> &tab, std::vector<TabType> &types);
 
-// SplineEvaluate on the interval holding r (first knot >= r, stepped back
-// unless r sits on it; the last knot takes the last interval); dout, when
+// SplineEvaluate's cubic at r, j the first knot >= r: the interval is stepped back
+// unless r sits on the knot; the last knot takes the last interval.  dout, when
 // given, receives the cubic's derivative.
-__device__ __forceinline__ bool spline_at(const double *x, const double *y, const double *yd, int n, double r, double *out,
-                                          double *dout = nullptr)
+__device__ __forceinline__ void spline_cubic(const double *x, const double *y, const double *yd, int n, int j, double r,
+                                             double *out, double *dout = nullptr)
 {
-    if (!(r >= x[0] && r <= x[n - 1])) return false;
-    int lo = 0, hi = n;   // lower_bound
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (x[mid] < r) lo = mid + 1;
-        else hi = mid;
-    }
-    int j = lo;
     if (r < x[j]) j--;
     if (j > n - 2) j = n - 2;
     const double p1 = x[j];
@@ -47,6 +39,20 @@ __device__ __forceinline__ bool spline_at(const double *x, const double *y, cons
     const double t = r - p1;
     *out = ((A3 * t + A2) * t + A1) * t + A0;
     if (dout) *dout = (3.0 * A3 * t + 2.0 * A2) * t + A1;
+}
+
+// SplineEvaluate on the interval holding r
+__device__ __forceinline__ bool spline_at(const double *x, const double *y, const double *yd, int n, double r, double *out,
+                                          double *dout = nullptr)
+{
+    if (!(r >= x[0] && r <= x[n - 1])) return false;
+    int lo = 0, hi = n;   // lower_bound
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (x[mid] < r) lo = mid + 1;
+        else hi = mid;
+    }
+    spline_cubic(x, y, yd, n, lo, r, out, dout);
     return true;
 }
 
