@@ -199,6 +199,7 @@ def scf_section(d, name, mode, max_iter, budget_s, verbose=False):
         chosen_cfg = {"batch": list(Ic.batch), "gather_trip": list(Ic.gather_trip), "workgroup": list(Ic.workgroup)}
     de = lambda e: abs(e - ref["e_total"]) / I.nAtoms
     plain_wall = ref["report_wall_s"]
+    gather = "matrix-core" if Ic.gather_trip[1] >= 4 else "vector-ALU"
     kmix = f"Kerker-preconditioned Pulay (k0 = {KERKER_K0:g}/bohr, mixing {KERKER_MIX:g})"
     out = {
         "workload": f"periodic cell {I.rank_box[3]}x{I.rank_box[4]}x{I.rank_box[5]} = {I.n_nodes} nodes, "
@@ -206,6 +207,8 @@ def scf_section(d, name, mode, max_iter, budget_s, verbose=False):
         "tol": SCF_TOL,
         "plain_fp64_kerker": {
             "form": f"FP64 Lanczos, one-node kernel, {kmix}, steps launched one by one", **plain_cfg,
+            "note": "the reference's loop structure; an FP64 SCF as the library runs it (resident kernel, step graph) "
+                    "is recorded in profiles/scf_c128_summary.md",
             "reference_tol": SCF_TOL_REF, **{k: ref[k] for k in keep},
             "at_common_stop": {"iterations": ref["report_iterations"], "wall_s": plain_wall,
                                "e_total": ref["report_e_total"],
@@ -217,7 +220,7 @@ def scf_section(d, name, mode, max_iter, budget_s, verbose=False):
                     "(python -m sqminiapp_amd.scf_run --config C128 --precision fp64 --mixing deck --max-iter 30); "
                     "recorded in profiles/scf_c128_summary.md, not repeated here"},
         "chosen_form": {
-            "form": f"FP32 Lanczos, batched kernel (MFMA projector gather), {kmix}, SCF step replayed from one captured "
+            "form": f"FP32 Lanczos, batched kernel ({gather} projector gather), {kmix}, SCF step replayed from one captured "
                     f"graph, " + ("start from the learned initial density (BF16 network inference)" if learned
                                    else "superposed atoms (no network weights found)"),
             **chosen_cfg, **{k: rc[k] for k in keep}, "guess_s": t_guess, "wall_with_guess_s": rc["wall_s"] + t_guess,

@@ -179,7 +179,7 @@ int sq_tridiag_nodes_weights_noalloc(sq_ctx *ctx, const double *diag, const doub
 int sq_density_fermi_energy(sq_ctx *ctx, double nelec, double beta, double *lambda_f, double *rho,
                             double *e_band, double *minus_ts);
 
-/* Per-node early exit of the batched Lanczos (the column-marching kernel): a
+/* Per-node early exit of the Lanczos passes (not in the generic kernel): a
  * node stops at n Lanczos steps once the lowest 8 Matsubara terms
  * (2/beta) g(lambda_f + i (2m+1) pi / beta), g(z) = e1^T (z - T_n)^{-1} e1,
  * of its Gauss rule change by less than tol between checks at n = min_steps,

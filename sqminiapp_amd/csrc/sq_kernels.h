@@ -148,7 +148,6 @@ int mlp_param_count(int K, int H);
 // overflow: device int counting points with more neighbours than the kernel holds
 hipError_t launch_mlp_features(const double4 *img, int nimg, const int G[3], const double h[3], const double R[3], int K,
                                double rf, float *out, int *overflow, hipStream_t st);
-// Z1, Z2 (may be null): pre-activations of the two hidden layers, for the deltas
 // The superposed atomic densities of a cell (unscaled), as build_atomic_density forms them on
 // the host: images in order; per type n knots, values and slopes from tab + off on.  *status: 3
 // where a radius lies below a table.
@@ -161,6 +160,7 @@ hipError_t launch_guess_add(double *rho, const float *y, const double *sum, doub
                             hipStream_t st);
 // rho *= ne / (sum dV), where that is positive
 hipError_t launch_guess_scale(double *rho, const double *sum, double ne, double dV, long n, hipStream_t st);
+// Z1, Z2 (may be null): pre-activations of the two hidden layers, for the deltas
 hipError_t launch_mlp_forward(const float *X, long N, const float *P, const float *mean, const float *rstd, float *H1,
                               float *H2, float *Z1, float *Z2, float *Y, int bf16, hipStream_t st);
 hipError_t launch_mlp_deltas(const float *Z1, const float *Z2, const float *Y, const float *T, long N, const float *P,

@@ -261,7 +261,7 @@ __device__ __forceinline__ void rotation(double f, double g, double &r, double &
 // off-diagonal, which the reference repeats from l on after every sweep, is
 // made inside the sweep, where d and e become final; a scan before each sweep
 // and the operators in place of rotation() took 13.3 ms for 16384 x n = 80, which
-// take 3.8 now.  The rows d, e and z lie in LDS (ql_kernel) or, for batches of which
+// take 3.4 to 3.8 now.  The rows d, e and z lie in LDS (ql_kernel) or, for batches of which
 // LDS holds only a part at a time, in device memory (ql_kernel_mem); ql_lanes.
 
 // Tridiagonals t0 .. t0 + mine - 1, one a lane; d, e and z of lane k at
@@ -451,8 +451,9 @@ __device__ __forceinline__ void occupation_block(const double *lam, const double
 // it -- and then counts at the new midpoint.  Count k leaves its state at state[k
 // & 1] and its partials in the (k + 2) % 3-th of three places: no block of a launch
 // writes what another still reads.  count: -2 at the lower end, -1 at the upper
-// end, then 0 (brackets, first midpoint), 1, ...  A halving takes 5 us; the count,
-// its sum and a look by the host took 60, on the device 16 in two launches.
+// end, then 0 (brackets, first midpoint), 1, ...  A halving takes 5 us where a rule
+// set is small, 8 and 11 for the rules of 7872 and 15744 grid nodes; the count, its sum and
+// a look by the host took 60, on the device 16 in two launches.
 __global__ void __launch_bounds__(kRedThreads) fermi_count(const double *lam, const double *w, long nq, double beta,
                                                            double nelec, const double *range, int count, BisState *state,
                                                            double *partial)

@@ -1,7 +1,7 @@
 // sq_resident.hip -- the resident Lanczos kernel (FP64): one workgroup runs the whole recurrence of one grid node with its Lanczos
 // vectors on chip; one thread owns one (x,y) column of the cube.
 //   v      the current vector: the lower nl planes in LDS, the rest in a slice
-//          of scratch that stays in the L2;
+//          of scratch (29^3: 17 of 29 planes);
 //   r      the previous vector, then the vector being built: the thread's whole
 //          column in registers, indexed statically (the z loops are unrolled to
 //          NZ planes and guarded by the cube's nz).
@@ -16,8 +16,9 @@
 // What it replaces: the batched kernel streams its vectors (B x 195 KB in FP64)
 // through the Infinity Cache and moved 5.4 TB/s past the L2, the rate a plain
 // copy reaches (5.1 TB/s), so the pass was bound by that
-// traffic; here only projector tables, the diagonal and the few planes that do
-// not fit cross the L2.
+// traffic; here projector tables, the diagonal and the planes that do not fit LDS
+// cross the L2 (29^3: 578 KB a node and step, 3.0 vectors where the batched kernel moves
+// 13.8; the scratch planes are written past it every step).
 //
 // Projector tables: radial pairs (t0, t2) of each image's box trimmed to the
 // reach of the radial functions, with kResPad zero planes below and above, so
