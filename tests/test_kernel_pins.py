@@ -5,7 +5,7 @@ kernel left out altogether."""
 import numpy as np
 import pytest
 
-from conftest import KERNEL_ENV, MG1
+from conftest import KERNEL_ENV, MG1, write_variant
 
 import sqminiapp_amd as sq
 
@@ -56,3 +56,29 @@ def test_resident_kernel_by_default_and_by_name(monkeypatch):
     named, planes_named, info_named = _run(monkeypatch, SQ_BATCH="0")
     assert planes > 0 and planes_named == planes and info == info_named == (0, 512, 0)   # 21^3: 441 columns
     assert np.array_equal(ab[0], named[0]) and np.array_equal(ab[1], named[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wg", ["512", "1024"])
+def test_one_node_kernel_stops_early_as_a_shorter_run(monkeypatch, tmp_path, wg):
+    """FP64 in the pinned one-node kernel: a node that stops equals a fixed run of its length."""
+    deck = write_variant(str(tmp_path), "L", nqp=40)
+    for k in KERNEL_ENV + ("SQ_NO_RESIDENT",):
+        monkeypatch.delenv(k, raising=False)
+    monkeypatch.setenv("SQ_ZMARCH_WG", wg)
+    with sq.Context(*deck) as c:
+        assert c.resident_planes() == 0 and c.info.batch[0] == 1 and c.info.workgroup[0] == int(wg)
+        c.run(sq.SQ_NL_KB, sq.SQ_FP64)
+        lf = c.density_fermi_energy()[0]
+        c.set_early_exit(1e-3, lf, 0.0, 12, 4)
+        c.run(sq.SQ_NL_KB, sq.SQ_FP64)
+        lam, w, _, _ = c.results()
+        sizes = c.rule_sizes()
+    assert sizes.min() >= 12 and np.any(sizes < 40)
+    for s in sorted(set(sizes.tolist()))[:2]:
+        with sq.Context(*deck, nqp=int(s)) as cs:
+            for i in np.nonzero(sizes == s)[0][:3]:
+                cs.run(sq.SQ_NL_KB, sq.SQ_FP64, begin=int(i), count=1)
+                ls, ws, _, _ = cs.results()
+                assert np.array_equal(lam[i, :s], ls[0]) and np.array_equal(w[i, :s], ws[0]), (i, s)
+                assert np.all(w[i, s:] == 0.0)
